@@ -241,6 +241,80 @@ __device__ __forceinline__ uint64_t special64(uint64_t x) {
     return (((x - 0x20 * ONES) & ~x) | ((q - ONES) & ~q) | ((b - ONES) & ~b)) & (0x80 * ONES);
 }
 
+// ------------------------------------------------------- reading JSON
+__device__ __forceinline__ int hexval(int c) {
+    const uint32_t d = (uint32_t)c - '0', a = ((uint32_t)c | 0x20) - 'a';  // 'A'-'F' fold onto 'a'-'f'
+    return d < 10 ? (int)d : a < 6 ? (int)a + 10 : -1;
+}
+// UTF-8 bytes of code point cp, packed little endian; *k = count
+__device__ __forceinline__ uint32_t utf8_pack(uint32_t cp, int *k) {
+    if (cp < 0x80) { *k = 1; return cp; }
+    if (cp < 0x800) { *k = 2; return (0xC0 | (cp >> 6)) | ((0x80 | (cp & 63)) << 8); }
+    if (cp < 0x10000) {
+        *k = 3;
+        return (0xE0 | (cp >> 12)) | ((0x80 | ((cp >> 6) & 63)) << 8) | ((0x80 | (cp & 63)) << 16);
+    }
+    *k = 4;
+    return (0xF0 | (cp >> 18)) | ((0x80 | ((cp >> 12) & 63)) << 8) | ((0x80 | ((cp >> 6) & 63)) << 16) |
+           ((0x80u | (cp & 63)) << 24);
+}
+
+// Four hex digits (bytes 0..3 of x) as a code unit, or -1.
+__device__ __forceinline__ int hex4(uint32_t x) {
+    uint32_t cu = 0;
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int h = hexval((int)((x >> (8 * j)) & 0xFF));
+        ok &= h >= 0;
+        cu = cu * 16 + (uint32_t)(h & 15);
+    }
+    return ok ? (int)cu : -1;
+}
+
+// Bit 7 of the first byte of x that is '"', '\\', below 0x20 or above 0x7F
+// (bits above it may be set too: borrows only run upwards from a byte that
+// is flagged itself).
+__device__ __forceinline__ uint64_t str_stop8(uint64_t x) {
+    constexpr uint64_t ONE = 0x0101010101010101ull;
+    const uint64_t q = x ^ (0x22 * ONE), b = x ^ (0x5C * ONE);
+    return (((q - ONE) & ~q) | ((b - ONE) & ~b) | (x - 0x20 * ONE) | x) & (0x80 * ONE);
+}
+// The same for '"' and '\\' only.
+__device__ __forceinline__ uint64_t quote_bs8(uint64_t x) {
+    constexpr uint64_t ONE = 0x0101010101010101ull;
+    const uint64_t q = x ^ (0x22 * ONE), b = x ^ (0x5C * ONE);
+    return (((q - ONE) & ~q) | ((b - ONE) & ~b)) & (0x80 * ONE);
+}
+// Continuation bytes a UTF-8 lead byte c takes under jackson's lead classes
+// (C0-DF one, E0-EF two, F0-F7 three), given x = the 8 bytes from the lead
+// byte on; 0 if c is no lead byte (a control, a stray continuation byte,
+// F8-FF) or a continuation byte is missing.
+__device__ __forceinline__ uint32_t utf8_extra(uint32_t c, uint64_t x) {
+    const uint32_t extra = (uint32_t)(c >= 0xC0) + (uint32_t)(c >= 0xE0) + (uint32_t)(c >= 0xF0);
+    const uint64_t msk = (1ull << (8 * extra)) - 1;
+    const uint64_t cb = (x >> 8) & msk & (0xC0C0C0ull);
+    const bool ok = c >= 0xC0 && c <= 0xF7 && cb == (0x808080ull & msk);
+    return ok ? extra : 0u;
+}
+
+// bit 7 of each byte set iff that byte is not an ASCII digit
+__device__ __forceinline__ uint64_t nondigit8(uint64_t x) {
+    const uint64_t m7 = 0x7F7F7F7F7F7F7F7Full;
+    const uint64_t ge0 = ((x & m7) + 0x5050505050505050ull) | x;   // >= '0' (or >= 0x80)
+    const uint64_t ge9 = ((x & m7) + 0x4646464646464646ull) | x;   // >= ':' (or >= 0x80)
+    return (~ge0 | ge9) & 0x8080808080808080ull;
+}
+
+// value of m (1..8) ASCII digits packed little endian in x (first digit low)
+__device__ __forceinline__ uint64_t digits8(uint64_t x, int m) {
+    uint64_t y = x - 0x3030303030303030ull;
+    if (m < 8) y <<= 8 * (8 - m);
+    y = (y * 10 + (y >> 8)) & 0x00FF00FF00FF00FFull;
+    y = (y * 100 + (y >> 16)) & 0x0000FFFF0000FFFFull;
+    return (y * 10000 + (y >> 32)) & 0xFFFFFFFFull;
+}
+
 // Direct global writes of a byte stream that starts at any offset.
 // Bytes gather in a 64-bit accumulator that always describes an aligned
 // output dword; full dwords are stored whole, and the first dword (shared

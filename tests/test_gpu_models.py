@@ -203,3 +203,41 @@ def test_model_decode_tape_and_reparse_match_oracle(codec, monkeypatch, tape):
     for fmt in (pj.FORMAT_ARRAY, pj.FORMAT_PRETTY):
         data = orc.encode_model(cols, fmt, pj.INCLUDE_ALWAYS)
         same_decode(codec, pj.MODEL_ORDER, data, array=True)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 127, 128, 129, 300])
+@pytest.mark.parametrize("span", [None, 32240, 32255, 32256, 32257, 40000])
+def test_model_decode_fast_path_edges(codec, n, span):
+    """The fast path at its edges, against the oracle: every subset of absent
+    properties, integers at their types' limits and beyond, every place of a
+    stop byte (escape, surrogate pair, multi-byte character) in a string read
+    16 bytes at a time, null and empty values; blocks of 128 records whose
+    bytes just fit the LDS tile of 32,256 or just do not (`span`: the bytes of
+    a full block), and blocks that are not full."""
+    ints = ["0", "-0", "7", "-1", "2147483647", "2147483648", "-2147483648", "-2147483649", "12345678", "123456789",
+            "1234567890123456", "12345678901234567", "9223372036854775807", "9223372036854775808",
+            "-9223372036854775808", "-9223372036854775809", "99999999999999999999", "01", "1.0", "1e2", "null"]
+    stops = ["", '\\"', "\\\\", "\\u00e9", "\\ud83d\\ude00", "\\ud83d", "é", "€", "\U0001f600", "\\x", "\\u12"]
+    orders, users = [], []
+    for i in range(n):
+        s = lambda k: '"' + "a" * ((i + 3 * k) % 34) + stops[(i // 3 + k) % len(stops)] + "b" * ((i * 7 + k) % 19) + '"'
+        big, small = ints[i % len(ints)], ints[(i * 5 + 2) % 9]
+        props = [("id", small if i % 4 else big), ("petId", ints[(i + 4) % 5]), ("quantity", ints[(i * 3) % 7]),
+                 ("shipDate", ["null", '""', s(0)][i % 3]),
+                 ("status", ['"placed"', '"approved"', '"delivered"', "null", '"placed"', '"placed "'][i % 6 if i % 11 else 4]),
+                 ("complete", ["true", "false", "null", "tru"][i % 4 if i % 13 == 0 else i % 3])]
+        orders.append("{" + ",".join(f'"{k}":{v}' for j, (k, v) in enumerate(props) if i & (1 << j) or i % 5 == 0) + "}")
+        props = [("id", small), ("username", s(1)), ("firstName", s(2)), ("lastName", '""'), ("email", s(3)),
+                 ("password", "null"), ("phone", s(4)), ("userStatus", ints[i % 7])]
+        users.append("{" + ",".join(f'"{k}":{v}' for j, (k, v) in enumerate(props) if (i * 37) & (1 << j) or i % 3 == 0) + "}")
+    for model, recs in ((pj.MODEL_ORDER, orders), (pj.MODEL_USER, users)):
+        lines = [r.encode("utf-8") for r in recs]
+        if span is not None:
+            # the first record of every block pads it out (a known string property where the model has one free)
+            for b in range(0, len(lines), 128):
+                blk = lines[b: b + 128]
+                want = span - sum(len(x) + 1 for x in blk[1:])
+                key = b'{"shipDate":"' if model == pj.MODEL_ORDER else b'{"username":"'
+                lines[b] = key + b"p" * max(0, want - len(key) - 3) + b'"}'
+        same_decode(codec, model, b"\n".join(lines) + b"\n")
+        same_decode(codec, model, b"[" + b",".join(lines) + b"]", array=True)
