@@ -241,3 +241,37 @@ def test_model_decode_fast_path_edges(codec, n, span):
                 lines[b] = key + b"p" * max(0, want - len(key) - 3) + b'"}'
         same_decode(codec, model, b"\n".join(lines) + b"\n")
         same_decode(codec, model, b"[" + b",".join(lines) + b"]", array=True)
+
+
+@pytest.mark.parametrize("fmt", [pj.FORMAT_ARRAY, pj.FORMAT_NDJSON, pj.FORMAT_PRETTY])
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 1030])
+def test_model_encode_tile_runs_match_oracle(codec, n, fmt):
+    """Blocks of 512 records leave through a tile of 79,872 bytes in runs of
+    whole records: blocks that need one run, several runs and runs of one
+    record, a record that fills the tile to the byte, is one byte longer or
+    much larger (at a block's start, end and alone), and the output cut at
+    and inside the runs."""
+    for size in (None, 60, 400, 2500):
+        recs = [{"id": i, "username": "u" * (0 if size is None else (i * 37) % size), "phone": 'q"\n\x01' * (i % 3),
+                 "userStatus": None if i % 4 else -i} for i in range(n)]
+        for k, big in ((0, 79872), (n - 1, 79873), (n // 2, 200_000), (n // 3, 79871)):
+            if size == 400:
+                recs[k] = {"username": "z" * (big - len('{"username":""}') - (2 if fmt == pj.FORMAT_PRETTY else 1))}
+        cols = to_model_columns(pj.MODEL_USER, recs)
+        ref = orc.encode_model(cols, fmt)
+        dev = cols.to_device()
+        out = torch.full((len(ref) + 64,), 0xEE, dtype=torch.uint8, device="cuda")
+        got = codec.encode_model(dev, fmt, out=out)
+        assert got.cpu().numpy().tobytes() == ref, (n, size)
+        assert (out[len(ref):].cpu().numpy() == 0xEE).all()
+        for cap in (len(ref) - 1, len(ref) // 2, 1):
+            if not 0 < cap < len(ref):
+                continue
+            out.fill_(0xEE)
+            with pytest.raises(pj.PetJsonError) as ei:
+                codec.encode_model(dev, fmt, out=out[:cap])
+            assert ei.value.status == pj.PJ_ERR_CAPACITY
+            host = out.cpu().numpy()
+            assert (host[cap:] == 0xEE).all()
+            w = host[:cap] != 0xEE
+            assert (host[:cap][w] == np.frombuffer(ref, np.uint8)[:cap][w]).all()
