@@ -47,6 +47,52 @@ __device__ __forceinline__ uint32_t lt_bytes4(uint32_t x, uint32_t c) {
 // bit i set iff bit 7 of byte i of m is set (m holds only bits 7, 15, 23, 31)
 __device__ __forceinline__ uint32_t movemask4(uint32_t m) { return (((m >> 7) * 0x00204081u) >> 21) & 0xFu; }
 
+// The bit planes of a 64-byte word: bit i of b[p] is bit p of byte i.  Any
+// class of bytes is then a few logic operations over all 64 bytes at once.
+// Built from the word's 16 dwords by byte permutes (byte j of row k becomes
+// byte 8 j + k of a 32-byte half) and three rounds of 8 x 8 bit transposes:
+// 128 vector operations per word, and about six per class after it, against
+// about 190 per class for a zero-byte test and a movemask per dword (array
+// frame of 1M records, 274 MB: k_arr_frame 264 -> 162 us, k_arr_sum 99 -> 83).
+struct Planes {
+    uint64_t b[8];
+};
+// m selects from x, ~m from y
+__device__ __forceinline__ uint32_t bitsel(uint32_t m, uint32_t x, uint32_t y) { return (x & m) | (y & ~m); }
+__device__ __forceinline__ void planes32(const uint32_t *w, uint32_t (&d)[8]) {
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+        const uint32_t w0 = w[g], w1 = w[2 + g], w2 = w[4 + g], w3 = w[6 + g];
+        const uint32_t l01 = __builtin_amdgcn_perm(w1, w0, 0x05010400u), h01 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
+        const uint32_t l23 = __builtin_amdgcn_perm(w3, w2, 0x05010400u), h23 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+        d[4 * g] = __builtin_amdgcn_perm(l23, l01, 0x05040100u);
+        d[4 * g + 1] = __builtin_amdgcn_perm(l23, l01, 0x07060302u);
+        d[4 * g + 2] = __builtin_amdgcn_perm(h23, h01, 0x05040100u);
+        d[4 * g + 3] = __builtin_amdgcn_perm(h23, h01, 0x07060302u);
+    }
+    constexpr uint32_t M[3] = {0x0F0F0F0Fu, 0x33333333u, 0x55555555u};
+#pragma unroll
+    for (int st = 0; st < 3; st++) {
+        const int D = 4 >> st;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            if (k & D) continue;
+            const uint32_t x = d[k], y = d[k + D];
+            d[k] = bitsel(M[st], x, y << D);
+            d[k + D] = bitsel(M[st], x >> D, y);
+        }
+    }
+}
+__device__ __forceinline__ Planes byte_planes(const uint32_t (&w)[16]) {
+    uint32_t lo[8], hi[8];
+    planes32(w, lo);
+    planes32(w + 8, hi);
+    Planes P;
+#pragma unroll
+    for (int p = 0; p < 8; p++) P.b[p] = (uint64_t)hi[p] << 32 | lo[p];
+    return P;
+}
+
 __device__ __forceinline__ uint64_t prefix_xor(uint64_t x) {
     x ^= x << 1; x ^= x << 2; x ^= x << 4; x ^= x << 8; x ^= x << 16; x ^= x << 32;
     return x;
@@ -211,8 +257,7 @@ __device__ __forceinline__ FS fs_cat(const FS &f, const FS &g) {
 struct AMasks {
     uint64_t q, b, o, c, m, nw;     // '"', '\\', '[' '{', ']' '}', ',', not whitespace
 };
-__device__ __forceinline__ AMasks arr_masks(const uint8_t *g, uint64_t avail) {
-    uint32_t w[16];
+__device__ __forceinline__ void arr_load(const uint8_t *g, uint64_t avail, uint32_t (&w)[16]) {
     if (avail >= 64) {
         const uint4 *q4 = reinterpret_cast<const uint4 *>(g);
 #pragma unroll
@@ -222,22 +267,29 @@ __device__ __forceinline__ AMasks arr_masks(const uint8_t *g, uint64_t avail) {
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; k++) w[k] = 0;
-        for (uint32_t j = 0; j < avail; j++) w[j >> 2] |= (uint32_t)g[j] << (8 * (j & 3));
+        for (int k = 0; k < 16; k++) {
+            w[k] = 0;
+            for (uint32_t j = 0; j < 4; j++)
+                if (4u * k + j < avail) w[k] |= (uint32_t)g[4 * k + j] << (8 * j);
+        }
     }
-    AMasks M{0, 0, 0, 0, 0, 0};
-    uint64_t ws = 0;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-        const uint32_t x = w[k], lx = x | 0x20202020u;
-        M.q |= (uint64_t)zero_bytes4(x ^ 0x22222222u) << (4 * k);
-        M.b |= (uint64_t)zero_bytes4(x ^ 0x5C5C5C5Cu) << (4 * k);
-        M.o |= (uint64_t)zero_bytes4(lx ^ 0x7B7B7B7Bu) << (4 * k);      // '[' or '{'
-        M.c |= (uint64_t)zero_bytes4(lx ^ 0x7D7D7D7Du) << (4 * k);      // ']' or '}'
-        M.m |= (uint64_t)zero_bytes4(x ^ 0x2C2C2C2Cu) << (4 * k);
-        ws |= (uint64_t)(zero_bytes4(x ^ 0x20202020u) | zero_bytes4(x ^ 0x09090909u) | zero_bytes4(x ^ 0x0D0D0D0Du) |
-                         zero_bytes4(x ^ 0x0A0A0A0Au)) << (4 * k);
-    }
+}
+__device__ __forceinline__ AMasks arr_masks(const uint32_t (&w)[16], uint64_t avail) {
+    const Planes B = byte_planes(w);
+    const uint64_t *b = B.b;
+    AMasks M;
+    const uint64_t hi2 = ~b[7] & ~b[6] & b[5] & ~b[4];                  // 0x2_
+    const uint64_t hi57 = ~b[7] & b[6] & b[4];                          // 0x5_ or 0x7_
+    const uint64_t lo_c = b[3] & b[2] & ~b[1] & ~b[0];
+    M.q = hi2 & ~b[3] & ~b[2] & b[1] & ~b[0];                           // 0x22
+    M.m = hi2 & lo_c;                                                   // 0x2C
+    M.b = hi57 & ~b[5] & lo_c;                                          // 0x5C
+    M.o = hi57 & b[3] & ~b[2] & b[1] & b[0];                            // 0x5B or 0x7B
+    M.c = hi57 & b[3] & b[2] & ~b[1] & b[0];                            // 0x5D or 0x7D
+    const uint64_t sp = hi2 & ~b[3] & ~b[2] & ~b[1] & ~b[0];            // 0x20
+    const uint64_t nine = ~b[7] & ~b[6] & ~b[5] & ~b[4] & b[3] &        // 0x09, 0x0A, 0x0D
+                          ((~b[2] & (b[1] ^ b[0])) | (b[2] & ~b[1] & b[0]));
+    const uint64_t ws = sp | nine;
     M.nw = ~ws & (avail >= 64 ? ~0ull : ((1ull << avail) - 1));
     return M;
 }
@@ -293,16 +345,24 @@ __device__ __forceinline__ FS block_fs_scan(FS v, FS *sh) {
     }
     return v;
 }
-// Summary of each block of BT * R words (thread t: words t R .. t R + R - 1).
-template <int BT, int R>
+// Summary of each block of BT * R words (thread t: words t R .. t R + R - 1,
+// the loads of ARR_U words, one 128-byte line, in flight together).
+template <int BT, int R, int ARR_U = (R > 1 ? 2 : 1)>
 __global__ __launch_bounds__(BT) void k_arr_sum(DecParams P) {
     __shared__ FS sh[BT];
     const uint32_t t = threadIdx.x;
     const uint64_t b = blockIdx.x, w0 = (b * BT + t) * R;
     FS acc = fs_id();
-    for (int r = 0; r < R; r++) {
-        const uint64_t w = w0 + r;
-        if (w < P.nblk64) acc = fs_cat(acc, word_fs(arr_masks(P.in + 64 * w, P.len - 64 * w)));
+    for (int r = 0; r < R; r += ARR_U) {
+        uint32_t x[ARR_U][16];
+#pragma unroll
+        for (int u = 0; u < ARR_U; u++)
+            if (w0 + r + u < P.nblk64) arr_load(P.in + 64 * (w0 + r + u), P.len - 64 * (w0 + r + u), x[u]);
+#pragma unroll
+        for (int u = 0; u < ARR_U; u++) {
+            const uint64_t w = w0 + r + u;
+            if (w < P.nblk64) acc = fs_cat(acc, word_fs(arr_masks(x[u], P.len - 64 * w)));
+        }
     }
     acc = block_fs_scan<BT>(acc, sh);
     if (t == BT - 1) P.arr_bsum[b] = acc;
@@ -332,7 +392,7 @@ __global__ __launch_bounds__(BT) void k_arr_scan(DecParams P, uint64_t nb) {
 // look-back of the counts), the first byte whose close brings the depth to
 // 0, and the first and last bytes that are not whitespace (one atomic per
 // block each).
-template <int BT, int R>
+template <int BT, int R, int ARR_U = (R > 1 ? 2 : 1)>
 __global__ __launch_bounds__(BT) void k_arr_frame(DecParams P) {
     __shared__ uint64_t sh_scan[BT / 64];
     __shared__ uint64_t sh_blk, sh_pre, sh_mn[3];
@@ -359,31 +419,42 @@ __global__ __launch_bounds__(BT) void k_arr_frame(DecParams P) {
     {
         uint32_t st = st0;
         int32_t dep = dep0;
+        uint32_t x[ARR_U][16];
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const uint64_t w = w0 + r;
-            if (w >= P.nblk64) break;
-            const AMasks M = arr_masks(P.in + 64 * w, P.len - 64 * w);
-            const AWord a = arr_word(M, st);
-            for (uint64_t m = a.md; m; m &= m - 1) {
-                const uint32_t i = (uint32_t)__builtin_ctzll(m);
-                if (dep + depth_at(a, i) == 1) sep[r] |= 1ull << i;
+            if (r % ARR_U == 0) {
+#pragma unroll
+                for (int u = 0; u < ARR_U; u++)
+                    if (w + u < P.nblk64) arr_load(P.in + 64 * (w + u), P.len - 64 * (w + u), x[u]);
             }
-            cnt += (uint64_t)__builtin_popcountll(sep[r]);
-            if (close == ~0ull)
-                for (uint64_t m = a.cd; m; m &= m - 1) {
-                    const uint32_t i = (uint32_t)__builtin_ctzll(m);
-                    if (dep + depth_at(a, i) == 0) {
-                        close = 64 * w + i;
-                        break;
+            if (w < P.nblk64) {
+                const AMasks M = arr_masks(x[r % ARR_U], P.len - 64 * w);
+                const AWord a = arr_word(M, st);
+                // a comma is at depth 1, or a close reaches 0, only if the
+                // word's closes can bring the depth that low
+                if (dep - __builtin_popcountll(a.cd) <= 1) {
+                    for (uint64_t m = a.md; m; m &= m - 1) {
+                        const uint32_t i = (uint32_t)__builtin_ctzll(m);
+                        if (dep + depth_at(a, i) == 1) sep[r] |= 1ull << i;
                     }
+                    cnt += (uint64_t)__builtin_popcountll(sep[r]);
+                    if (close == ~0ull)
+                        for (uint64_t m = a.cd; m; m &= m - 1) {
+                            const uint32_t i = (uint32_t)__builtin_ctzll(m);
+                            if (dep + depth_at(a, i) == 0) {
+                                close = 64 * w + i;
+                                break;
+                            }
+                        }
                 }
-            if (M.nw) {
-                if (first == ~0ull) first = 64 * w + (uint64_t)__builtin_ctzll(M.nw);
-                lastp1 = 64 * w + 64 - (uint64_t)__builtin_clzll(M.nw);
+                if (M.nw) {
+                    if (first == ~0ull) first = 64 * w + (uint64_t)__builtin_ctzll(M.nw);
+                    lastp1 = 64 * w + 64 - (uint64_t)__builtin_clzll(M.nw);
+                }
+                dep += __builtin_popcountll(a.od) - __builtin_popcountll(a.cd);
+                st = a.out;
             }
-            dep += __builtin_popcountll(a.od) - __builtin_popcountll(a.cd);
-            st = a.out;
         }
     }
     if (first != ~0ull) atomicMin((unsigned long long *)&sh_mn[0], (unsigned long long)first);
@@ -2214,6 +2285,103 @@ __device__ __forceinline__ void tile_bitmaps(const uint8_t *tile, uint32_t nw, u
     }
 }
 
+// The same bitmaps built by one wave, lane l taking word 64 r + l in round r
+// (neighbouring lanes read neighbouring words).  The classes come from the
+// words' bit planes; what a word needs of the words before it (is its first
+// byte escaped, is it entered inside a string, how many continuation bytes
+// does it owe) crosses the lanes in ballots and one shuffle, and the rounds
+// in scalars.  Returns whether some bit of the bad-byte map is set among
+// bytes [lo, hi] (BAD only).  250,000 skewed lines (137 MB):
+// k_dec_measure_long 398 -> 226 us against per-dword movemasks with a run of
+// words per thread (bank conflicts) and a serial check of the map.
+template <bool BAD = true>
+__device__ __forceinline__ bool tile_bitmaps_wave(const uint8_t *tile, uint32_t nw, uint64_t *spec, uint64_t *badm,
+                                                  uint32_t lo, uint32_t hi) {
+    const uint32_t l = threadIdx.x & 63;
+    const uint64_t below = (1ull << l) - 1;
+    uint32_t ecarry = 0, scarry = 0, ucarry = 0;     // of the round before: escaped, in a string, bytes owed (bits)
+    bool any = false;
+    for (uint32_t r0 = 0; r0 < nw; r0 += 64) {
+        const uint32_t w = r0 + l;
+        uint32_t x[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = 0;
+        if (w < nw) {
+            const uint4 *q4 = reinterpret_cast<const uint4 *>(tile + 64 * w);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint4 v = q4[k];
+                x[4 * k] = v.x; x[4 * k + 1] = v.y; x[4 * k + 2] = v.z; x[4 * k + 3] = v.w;
+            }
+        }
+        const Planes PL = byte_planes(x);
+        const uint64_t *b = PL.b;
+        const uint64_t Q = ~b[7] & ~b[6] & b[5] & ~b[4] & ~b[3] & ~b[2] & b[1] & ~b[0];
+        const uint64_t B = ~b[7] & b[6] & ~b[5] & b[4] & b[3] & b[2] & ~b[1] & ~b[0];
+        // escaped characters: a word whose predecessor ends in a backslash
+        // learns from the composed carries whether its first byte is one
+        uint32_t c0, c1, cin = 0;
+        uint64_t E = escaped64(B, 0, &c0);
+        uint32_t eout = c0;
+        if (__ballot(c0 != 0) | ecarry) {
+            const uint64_t E1 = escaped64(B, 1, &c1);
+            uint32_t F = c0 | (c1 << 1);
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t G = (uint32_t)__shfl_up((int)F, (unsigned)d, 64);
+                if (l >= (uint32_t)d) F = ((F >> (G & 1)) & 1) | (((F >> ((G >> 1) & 1)) & 1) << 1);
+            }
+            const uint32_t Fp = (uint32_t)__shfl_up((int)F, 1u, 64);
+            cin = l == 0 ? ecarry : (Fp >> ecarry) & 1;
+            if (cin) E = E1;
+            eout = (F >> ecarry) & 1;
+        }
+        ecarry = (uint32_t)__builtin_amdgcn_readlane((int)eout, 63);
+        const uint64_t Qu = Q & ~E;
+        if (w < nw) spec[w] = B | Qu;
+        if constexpr (BAD) {
+            const uint64_t N = ~b[7] & ~b[6] & ~b[5] & ~b[4] & b[3] & ~b[2] & b[1] & ~b[0];
+            const uint64_t C = ~b[7] & ~b[6] & ~b[5];
+            // quote parity since the last newline; entered inside a string?
+            uint32_t par = (uint32_t)__builtin_popcountll(Qu) & 1;
+            if (N) {
+                const int last = 63 - __builtin_clzll(N);
+                par = last == 63 ? 0 : (uint32_t)__builtin_popcountll(Qu >> (last + 1)) & 1;
+            }
+            const uint64_t pm = __ballot(par != 0), nm = __ballot(N != 0), nb = nm & below;
+            const uint64_t since = nb ? ~0ull << (63 - __builtin_clzll(nb)) : ~0ull;
+            const uint32_t in = ((uint32_t)__builtin_popcountll(pm & below & since) + (nb ? 0u : scarry)) & 1;
+            uint64_t s = prefix_xor(Qu) ^ (in ? ~0ull : 0ull);
+            for (uint64_t m = N; m; m &= m - 1) {
+                const int p = __builtin_ctzll(m);
+                if ((s >> p) & 1) s ^= p == 63 ? 0ull : (~0ull << (p + 1));
+            }
+            scarry = (uint32_t)__builtin_amdgcn_readlane((N >> 63) ? 0 : (int)(s >> 63), 63);
+            uint64_t bad = C & s;
+            // UTF-8: lead bytes against the continuation bytes they owe
+            if (__ballot(b[7] != 0) | ucarry) {
+                const uint64_t h2 = b[7] & b[6], h3 = h2 & b[5], h4 = h3 & b[4];
+                const uint64_t cont = b[7] & ~b[6], l2 = h2 & ~b[5], l3 = h3 & ~b[4], l4 = h4 & ~b[3], badl = h4 & b[3];
+                const uint32_t owe = (uint32_t)((l2 >> 63) | (l3 >> 63) | (l3 >> 62) | (l4 >> 63) | (l4 >> 62) | (l4 >> 61));
+                const uint32_t up = (uint32_t)__shfl_up((int)owe, 1u, 64);
+                const uint64_t expect = (l2 << 1) | (l3 << 1) | (l3 << 2) | (l4 << 1) | (l4 << 2) | (l4 << 3) |
+                                        (l == 0 ? ucarry : up);
+                ucarry = (uint32_t)__builtin_amdgcn_readlane((int)owe, 63);
+                bad |= ((cont ^ expect) | badl) & (s | (s << 1) | in);
+            }
+            if (w < nw) {
+                badm[w] = bad;
+                uint64_t m = bad;
+                if (w < (lo >> 6) || w > (hi >> 6)) m = 0;
+                if (w == (lo >> 6)) m &= ~0ull << (lo & 63);
+                if (w == (hi >> 6)) m &= (hi & 63) == 63 ? ~0ull : ((2ull << (hi & 63)) - 1);
+                any |= m != 0;
+            }
+        }
+    }
+    return __ballot(any) != 0;
+}
+
 // ---------------------------------------------------------------- vector look-back
 // Per block PJ_DEC_NCNT words, one per counter, each holding its flag in the
 // top two bits (LB_AGG: block aggregate, LB_PRE: inclusive prefix) and the
@@ -2701,7 +2869,6 @@ __global__ __launch_bounds__(64) void k_dec_measure_long(DecParams P) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
     __shared__ uint64_t badm[TILE / 64 + 1];
-    __shared__ uint64_t sh_scan[1];
     const uint64_t cnt = *P.long_count, L = P.lines;
     const uint32_t t = threadIdx.x;
     for (uint64_t i = blockIdx.x; i < cnt; i += gridDim.x) {
@@ -2725,9 +2892,8 @@ __global__ __launch_bounds__(64) void k_dec_measure_long(DecParams P) {
             __syncthreads();
             if (P.array_doc && t == 0) tile[s0 + n] = '\n';
             __syncthreads();
-            tile_bitmaps<64>(tile, nw, spec, badm, sh_scan);
+            bad = tile_bitmaps_wave(tile, nw, spec, badm, s0, s0 + n);
             __syncthreads();
-            bad = line_bad(badm, nw, s0, n);
             if (bad) code = PJ_REC_STRING;          // provisional: k_dec_errcode settles it
             else {
                 code = fline_wave<false>((const PJ_LDS uint8_t *)tile, (const PJ_LDS uint64_t *)spec, s0, n, r, nullptr, nullptr);
@@ -2933,7 +3099,6 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
     __shared__ uint64_t badm[TILE / 64 + 1];
-    __shared__ uint64_t sh_scan[1];
     const uint64_t cnt = *P.long_count;
     if (!dec_room(P)) return;
     const pj_pet_columns &o = P.o;
@@ -2963,7 +3128,7 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
         __syncthreads();
         if (P.array_doc && threadIdx.x == 0) tile[gs + n - a0] = '\n';
         __syncthreads();
-        tile_bitmaps<64, false>(tile, nw, spec, badm, sh_scan);  // the line is valid: specials only
+        tile_bitmaps_wave<false>(tile, nw, spec, badm, 0, 0);  // the line is valid: specials only
         __syncthreads();
         const uint64_t pb = l / LPB;
         uint64_t base[PJ_DEC_NCNT];
@@ -3012,7 +3177,6 @@ __global__ __launch_bounds__(BT) void k_dec_errcode(DecParams P) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
     __shared__ uint64_t badm[TILE / 64 + 1];
-    __shared__ uint64_t sh_scan[1];
     __shared__ uint32_t sh_cut;
     const uint64_t cnt = *P.dq_count;
     const uint32_t t = threadIdx.x;
@@ -3036,7 +3200,8 @@ __global__ __launch_bounds__(BT) void k_dec_errcode(DecParams P) {
         if (P.array_doc && t == 0) tile[s0 + n] = '\n';
         if (t == 0) sh_cut = n;
         __syncthreads();
-        tile_bitmaps<BT>(tile, nw, spec, badm, sh_scan);
+        static_assert(BT == 64, "one wave builds the bitmaps");
+        tile_bitmaps_wave(tile, nw, spec, badm, s0, s0 + n);
         __syncthreads();
         // the first bad byte of the line
         for (uint32_t k = (s0 >> 6) + t; k <= ((s0 + n) >> 6) && k < nw; k += BT) {
@@ -3125,19 +3290,26 @@ hipError_t pj_launch_dec_index(const DecParams &P, hipStream_t st) {
     return hipGetLastError();
 }
 
-#ifndef PJ_ARR_R
-#define PJ_ARR_R 8
-#endif
-constexpr int ARR_BT = 256, ARR_R = PJ_ARR_R;
-uint64_t pj_arr_blocks(uint64_t nblk64) { return (nblk64 + ARR_BT * ARR_R - 1) / (ARR_BT * ARR_R); }
+// Words per thread of the frame kernels: eight for large documents, one for
+// those that eight would leave on fewer blocks than a few per CU (a page of
+// 20 records: k_arr_sum 24 -> 10 us, k_arr_frame 35 -> 12 us).
+constexpr int ARR_BT = 256, ARR_R = 8;
+constexpr uint64_t ARR_SMALL = (uint64_t)ARR_BT * 1024;     // words (16 MiB)
+uint64_t pj_arr_blocks(uint64_t nblk64) {
+    const uint64_t per = nblk64 <= ARR_SMALL ? ARR_BT : ARR_BT * ARR_R;
+    return (nblk64 + per - 1) / per;
+}
 uint64_t pj_arr_threads(uint64_t nblk64) { return pj_arr_blocks(nblk64) * ARR_BT; }
 
 hipError_t pj_launch_arr_frame(const DecParams &P, hipStream_t st) {
     const uint64_t g = pj_arr_blocks(P.nblk64);
+    const bool small = P.nblk64 <= ARR_SMALL;
     if (g) {                                        // an empty document has no frame: the verdict says so
-        hipLaunchKernelGGL((pj::k_arr_sum<ARR_BT, ARR_R>), dim3((unsigned)g), dim3(ARR_BT), 0, st, P);
+        hipLaunchKernelGGL((small ? pj::k_arr_sum<ARR_BT, 1> : pj::k_arr_sum<ARR_BT, ARR_R>), dim3((unsigned)g),
+                           dim3(ARR_BT), 0, st, P);
         hipLaunchKernelGGL((pj::k_arr_scan<1024>), dim3(1), dim3(1024), 0, st, P, g);
-        hipLaunchKernelGGL((pj::k_arr_frame<ARR_BT, ARR_R>), dim3((unsigned)g), dim3(ARR_BT), 0, st, P);
+        hipLaunchKernelGGL((small ? pj::k_arr_frame<ARR_BT, 1> : pj::k_arr_frame<ARR_BT, ARR_R>), dim3((unsigned)g),
+                           dim3(ARR_BT), 0, st, P);
     }
     hipLaunchKernelGGL(pj::k_arr_fin, dim3(1), dim3(1), 0, st, P);
     return hipGetLastError();
