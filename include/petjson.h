@@ -191,7 +191,8 @@ void        pj_default_options(pj_options *opt);
 pj_status   pj_set_options(pj_ctx *ctx, const pj_options *opt);
 /* Thread-local text of the last failure on this thread. */
 const char *pj_last_error(void);
-/* Duration (ms, HIP events on the context stream) of the last call's kernels:
+/* Duration (ms, device clock stamps at the start of each launch and of the
+ * one that ends the call) of the last call's kernels:
  * index 0 = whole device pipeline, 1.. = individual kernels in launch order.
  * Returns the number of entries written. */
 int         pj_last_timings(const pj_ctx *ctx, float *ms, int cap);

@@ -57,6 +57,7 @@ struct DevBuf {
 };
 
 constexpr int MAX_EV = 12;
+constexpr int BIG_RECENT = 16;
 
 // A copy engine between pageable host memory and the device: its own copy
 // stream, two pinned bounce buffers and their events.
@@ -92,8 +93,12 @@ struct pj_ctx {
     hipEvent_t seg_done[2] = {};      // streamed encode: a segment's bytes and length are final
     uint64_t *noalloc_scratch = nullptr;  // this device's fixed encode scratch (device address)
     bool flat_wide = false;       // flat encodes use the wide tile (records seen too long for the compact one)
-    bool big_seen = true;         // the last nested encode listed large records (k_enc_big gets a full grid)
-    hipEvent_t ev[MAX_EV] = {};
+    // nested encodes since one listed large records: while below BIG_RECENT,
+    // k_enc_big follows the pass without waiting for its count
+    int big_since = 1 << 20;
+    uint64_t scan_zero = 0;       // leading words of `scan` known to be zero (left so by the last encode)
+    uint64_t *stamps = nullptr;   // MAX_EV clock stamps of the call's launches (pinned, after the 64 result words)
+    double ticks_per_ms = 1e5;    // of the device's wall clock
     int n_ev = 0;
     float timings[MAX_EV] = {};
     int n_timings = 0;
@@ -107,24 +112,16 @@ pj_status bind(pj_ctx *c) {
     return PJ_OK;
 }
 
-pj_status mark(pj_ctx *c) {  // record the next timing event
-    if (c->n_ev < MAX_EV) PJ_HIP(hipEventRecord(c->ev[c->n_ev++], c->stream));
-    return PJ_OK;
-}
+// Where the next launch stamps its start (null past the last slot).
+uint64_t *mark(pj_ctx *c) { return c->n_ev < MAX_EV ? c->stamps + c->n_ev++ : nullptr; }
 
-pj_status finish_timing(pj_ctx *c) {
+// After the stream has drained: the intervals between the stamps.
+void finish_timing(pj_ctx *c) {
     c->n_timings = 0;
-    if (c->n_ev >= 2) {
-        PJ_HIP(hipEventSynchronize(c->ev[c->n_ev - 1]));
-        float ms = 0;
-        PJ_HIP(hipEventElapsedTime(&ms, c->ev[0], c->ev[c->n_ev - 1]));
-        c->timings[c->n_timings++] = ms;
-        for (int k = 1; k < c->n_ev && c->n_timings < MAX_EV; k++) {
-            PJ_HIP(hipEventElapsedTime(&ms, c->ev[k - 1], c->ev[k]));
-            c->timings[c->n_timings++] = ms;
-        }
-    }
-    return PJ_OK;
+    if (c->n_ev < 2) return;
+    auto ms = [&](int a, int b) { return (float)((double)(int64_t)(c->stamps[b] - c->stamps[a]) / c->ticks_per_ms); };
+    c->timings[c->n_timings++] = ms(0, c->n_ev - 1);
+    for (int k = 1; k < c->n_ev && c->n_timings < MAX_EV; k++) c->timings[c->n_timings++] = ms(k - 1, k);
 }
 
 // ---------------------------------------------------------------- host copies
@@ -281,6 +278,71 @@ pj_status d2h(pj_ctx *c, void *host, const void *dev, size_t n, hipEvent_t after
     return PJ_OK;
 }
 
+// Copies of at most SMALL_COPY bytes in all (SMALL_PINNED when the host side is
+// pinned, whose own DMA needs no bounce copy) go through the bounce buffers in
+// one launch on the context stream, 16 bytes per access straight from or to
+// the pinned memory: for a few pieces of a few KiB the copy calls, each with
+// its events and its wait, cost far more than the bytes (decode of a body of
+// 20 records, 17 columns out: 0.76 ms with them, 0.14 ms now).
+constexpr size_t SMALL_COPY = 4 << 20, SMALL_PINNED = 64 << 10;
+struct Piece {
+    void *dst;
+    const void *src;
+    uint64_t n;
+};
+inline uint64_t align16(uint64_t n) { return (n + 15) & ~15ull; }
+
+// Host bytes to the device ahead of the context stream's next work; small
+// inputs are only queued (the caller's next wait on the stream covers them).
+pj_status h2d_input(pj_ctx *c, void *dev, const void *host, size_t n) {
+    if (!n) return PJ_OK;
+    pj_status s = xfer_init(c->xin);
+    if (s) return s;
+    if (n > std::min(SMALL_COPY, c->xin.chunk & ~size_t(15)) || (n > SMALL_PINNED && pinned_host(host, n)))
+        return h2d(c, dev, host, n);
+    std::memcpy(c->xin.bounce[0], host, n);
+    CopyPieces C{};
+    C.dst[0] = static_cast<uint8_t *>(dev);
+    C.src[0] = c->xin.bounce[0];
+    C.n[0] = n;
+    C.k = 1;
+    PJ_HIP(pj_launch_copy_pieces(C, c->stream));
+    return PJ_OK;
+}
+
+// Pieces of device memory (16-byte aligned, readable to a multiple of 16
+// bytes; at most 20) to host memory, after the context stream's work.
+pj_status d2h_pieces(pj_ctx *c, const Piece *p, int k) {
+    pj_status s = xfer_init(c->xout);
+    if (s) return s;
+    uint64_t total = 0;
+    int big = 0;                             // the largest piece stands for all of them
+    for (int j = 0; j < k; j++) {
+        total += align16(p[j].n);
+        if (p[j].n > p[big].n) big = j;
+    }
+    if (total > std::min(SMALL_COPY, c->xout.chunk) || k > 20 ||
+        (total > SMALL_PINNED && pinned_host(p[big].dst, p[big].n))) {
+        for (int j = 0; j < k; j++)
+            if (p[j].n && (s = d2h(c, p[j].dst, p[j].src, p[j].n, nullptr, false))) return s;
+        return d2h_wait(c);
+    }
+    CopyPieces C{};
+    uint64_t off = 0;
+    for (int j = 0; j < k; j++) {
+        C.dst[j] = c->xout.bounce[0] + off;
+        C.src[j] = static_cast<const uint8_t *>(p[j].src);
+        C.n[j] = p[j].n;
+        off += align16(p[j].n);
+    }
+    C.k = k;
+    PJ_HIP(pj_launch_copy_pieces(C, c->stream));
+    PJ_HIP(hipStreamSynchronize(c->stream));
+    for (int j = 0; j < k; j++)
+        if (p[j].n) std::memcpy(p[j].dst, C.dst[j], p[j].n);
+    return PJ_OK;
+}
+
 bool nested_cols(const pj_pet_columns *c) { return c->cat_id || c->photo_off || c->tag_off; }
 uint64_t enc_big_cap() {
     if (const char *e = std::getenv("PETJSON_ENC_BIG_CAP")) return std::strtoull(e, nullptr, 10);
@@ -364,13 +426,11 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         const uint64_t len = format == PJ_FORMAT_ARRAY ? 2 : format == PJ_FORMAT_PRETTY ? 3 : 0;
         *out_len = len;
         if (!count_only && len && len <= cap) {
-            if ((s = mark(ctx))) return s;
             const uint32_t w = format == PJ_FORMAT_ARRAY ? '[' | (']' << 8) : '[' | (' ' << 8) | (']' << 16);
             PJ_HIP(pj_launch_put_bytes(out, w, (int)len, ctx->stream));
-            if ((s = mark(ctx))) return s;
         }
         PJ_HIP(hipStreamSynchronize(ctx->stream));
-        if ((s = finish_timing(ctx))) return s;
+        finish_timing(ctx);                                     // (no kernel worth timing: no entries)
         return len > cap && !count_only ? fail(PJ_ERR_CAPACITY, "output capacity too small") : PJ_OK;
     }
     const bool pretty = format == PJ_FORMAT_PRETTY;
@@ -397,6 +457,7 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     const bool defer_big = nested_cols(cols) && !pretty && !count_only && !fixed_scratch;
     const uint64_t big_cap = defer_big ? std::min<uint64_t>(n, enc_big_cap()) : 0;
     uint64_t *sc;
+    const void *sc_was = ctx->scan.p;
     std::unique_lock<std::mutex> noalloc_guard;
     if (fixed_scratch) {
         if (n > PJ_NOALLOC_MAX_RECORDS(nested_cols(cols)) || nblk + 4 + 128 > PJ_NOALLOC_SCRATCH_WORDS)
@@ -409,8 +470,20 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         noalloc_guard = std::unique_lock<std::mutex>(pj::noalloc_lock(ctx->device));
     } else {
         PJ_HIP(ctx->scan.ensure((nblk + 4 + 128 + (two_pass ? GEO_WORDS * nblk : 0) + 2 * big_cap) * sizeof(uint64_t)));
+        if (sc_was != ctx->scan.p) ctx->scan_zero = 0;
         sc = static_cast<uint64_t *>(ctx->scan.p);
     }
+    // the words a pass starts from zero: the last encode left them so, or a
+    // fill clears them (up to CLEAR_AFTER of them are cleared again as the
+    // results go out, which spares the next call the fill's launch)
+    constexpr uint64_t CLEAR_AFTER = 2048;
+    const uint64_t head = nblk + 4;
+    bool clean = !fixed_scratch && ctx->scan_zero >= head;
+    ctx->scan_zero = 0;
+    // k_enc_big runs behind the pass when a recent call listed large records;
+    // otherwise only once the pass's count says that there are some, after
+    // the wait for it (an empty launch costs a call of a page of records 10%)
+    const bool big_now = big_cap && (seg || two_pass || ctx->big_since < BIG_RECENT);
     EncParams P;
     std::memset(&P, 0, sizeof P);
     P.c = *cols;
@@ -442,42 +515,52 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     P.order_by_id = nested_cols(cols) || pretty || seg ? 0 : 1;
     P.spin_limit = spin_limit();
     for (int attempt = 0;; attempt++) {
-        if ((s = mark(ctx))) return s;
-        PJ_HIP(pj_launch_fill_u64(sc, nblk + 4, 0, ctx->stream));
-        if ((s = mark(ctx))) return s;
+        // (a segment of a streamed encode leaves the timings alone)
+        uint64_t *t0 = seg ? nullptr : mark(ctx), *t1 = seg ? nullptr : mark(ctx);
+        if (!clean) PJ_HIP(pj_launch_fill_u64(sc, head, 0, ctx->stream, t0));
+        P.stamp = t1;
         if (pretty_tiled) PJ_HIP(pj_launch_encode_pretty(P, ctx->stream));
         else if (pretty) PJ_HIP(pj_launch_encode_rows(P, true, ctx->stream));
         else if (two_pass) {
             P.geo = geo;
             PJ_HIP(pj_launch_encode_measure(P, ctx->stream));
             if (!count_only) {
-                if ((s = mark(ctx))) return s;
-                PJ_HIP(pj_launch_fill_u64(sc, 1, 0, ctx->stream));   // the writer's tickets
+                PJ_HIP(pj_launch_fill_u64(sc, 1, 0, ctx->stream, mark(ctx)));   // the writer's tickets
+                P.stamp = nullptr;
                 P.geo = geo;
                 PJ_HIP(pj_launch_encode(P, true, false, ctx->stream));
-                if (big_cap) PJ_HIP(pj_launch_encode_big(P, ctx->big_seen, ctx->stream));
+                if (big_now) PJ_HIP(pj_launch_encode_big(P, ctx->big_since < BIG_RECENT, ctx->stream));
             }
         } else {
             PJ_HIP(pj_launch_encode(P, nested_cols(cols), ctx->flat_wide, ctx->stream));
-            if (big_cap) PJ_HIP(pj_launch_encode_big(P, ctx->big_seen, ctx->stream));
+            if (big_now) PJ_HIP(pj_launch_encode_big(P, ctx->big_since < BIG_RECENT, ctx->stream));
         }
-        if ((s = mark(ctx))) return s;
         if (seg) {
             PJ_HIP(hipMemcpyAsync(seg->len, sc + 1, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
             PJ_HIP(hipEventRecord(seg->done, ctx->stream));
             return PJ_OK;
         }
-        PJ_HIP(hipMemcpyAsync(ctx->pinned, sc, 4 * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        const uint64_t clear = !fixed_scratch && head <= CLEAR_AFTER ? head : 0;
+        // (the large-record count stays until k_enc_big has read it)
+        PJ_HIP(pj_launch_publish(ctx->pinned, sc, 4, clear, big_cap && !big_now ? 3 : -1, ctx->stream, mark(ctx)));
         PJ_HIP(hipStreamSynchronize(ctx->stream));
-        if (!P.order_by_id || ctx->pinned[0] == 0 || attempt > 0) break;
+        if (clean) *t0 = *t1;                                   // no fill ran
+        const bool redo = P.order_by_id && ctx->pinned[0] != 0 && attempt == 0;
+        if (big_cap && !big_now && ctx->pinned[3]) {
+            ctx->n_ev--;                                        // the pass ends with its large records
+            PJ_HIP(pj_launch_encode_big(P, true, ctx->stream));
+            PJ_HIP(pj_launch_publish(ctx->pinned, sc, 0, 0, -1, ctx->stream, mark(ctx)));
+            PJ_HIP(hipStreamSynchronize(ctx->stream));
+        } else if (!redo) ctx->scan_zero = clear;
+        clean = false;
+        if (!redo) break;
         P.order_by_id = 0;                                      // redo in ticket order
         ctx->n_ev = 0;
     }
-    // the next nested encode's k_enc_big grid follows this one's large records
-    if (big_cap) ctx->big_seen = ctx->pinned[3] != 0;
+    if (big_cap) ctx->big_since = ctx->pinned[3] ? 0 : std::min(ctx->big_since + 1, 1 << 20);
     // flat records too long for the compact tile: later calls use the wide one
     if (!pretty && !nested_cols(cols) && !ctx->flat_wide && ctx->pinned[2] * 64 > nblk) ctx->flat_wide = true;
-    if ((s = finish_timing(ctx))) return s;
+    finish_timing(ctx);
     *out_len = ctx->pinned[1];
     if (!count_only && *out_len > cap) return fail(PJ_ERR_CAPACITY, "output capacity too small");
     return PJ_OK;
@@ -575,9 +658,15 @@ pj_ctx *pj_create(int device, pj_status *status) {
     pj_ctx *c = new pj_ctx();
     c->device = device;
     bool ok = hipSetDevice(device) == hipSuccess && hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess &&
-              hipHostMalloc((void **)&c->pinned, 64 * sizeof(uint64_t), hipHostMallocDefault) == hipSuccess &&
+              hipHostMalloc((void **)&c->pinned, (64 + MAX_EV) * sizeof(uint64_t), hipHostMallocDefault) == hipSuccess &&
               pj_noalloc_scratch_init(device, &c->noalloc_scratch) == hipSuccess;
-    for (int k = 0; ok && k < MAX_EV; k++) ok = hipEventCreate(&c->ev[k]) == hipSuccess;
+    int khz = 0;
+    ok = ok && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0;
+    if (ok) {
+        c->stamps = c->pinned + 64;
+        std::memset(c->stamps, 0, MAX_EV * sizeof(uint64_t));
+        c->ticks_per_ms = khz;
+    }
     if (!ok) {
         g_err = "context set-up failed";
         pj_destroy(c);
@@ -600,7 +689,6 @@ void pj_destroy(pj_ctx *c) {
     c->tape.release();
     c->seg_in[0].release();
     c->seg_in[1].release();
-    for (auto &e : c->ev) if (e) (void)hipEventDestroy(e);
     if (c->pinned) (void)hipHostFree(c->pinned);
     xfer_free(c->xin);
     xfer_free(c->xout);
@@ -646,6 +734,7 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
     // (ticket, total, look-back words), the selected indices
     const uint64_t w_sel = 2 + pj_select_blocks(n), w_enc = 2 + nblk;
     PJ_HIP(ctx->scan.ensure((w_sel + w_enc + n + 1) * sizeof(uint64_t)));
+    ctx->scan_zero = 0;
     uint64_t *sc = static_cast<uint64_t *>(ctx->scan.p), *ec = sc + w_sel, *sel = ec + w_enc;
     EncParams P;
     std::memset(&P, 0, sizeof P);
@@ -659,12 +748,11 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
         P.ticket = reinterpret_cast<unsigned long long *>(sc);
         P.total = sc + 1;
         P.state = sc + 2;
-        if ((s = mark(ctx))) return s;
-        PJ_HIP(pj_launch_fill_u64(sc, w_sel + w_enc, 0, ctx->stream));
-        if ((s = mark(ctx))) return s;
+        PJ_HIP(pj_launch_fill_u64(sc, w_sel + w_enc, 0, ctx->stream, mark(ctx)));
+        P.stamp = mark(ctx);
         PJ_HIP(pj_launch_select_status(P, status_mask, sel, ctx->stream));
-        if ((s = mark(ctx))) return s;
-        PJ_HIP(hipMemcpyAsync(ctx->pinned, sc + 1, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        P.stamp = nullptr;
+        PJ_HIP(pj_launch_publish(ctx->pinned, sc + 1, 1, 0, -1, ctx->stream, mark(ctx)));
         PJ_HIP(hipStreamSynchronize(ctx->stream));
         m = ctx->pinned[0];
     }
@@ -678,7 +766,7 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
             PJ_HIP(pj_launch_put_bytes(out, w, (int)len, ctx->stream));
         }
         PJ_HIP(hipStreamSynchronize(ctx->stream));
-        if ((s = finish_timing(ctx))) return s;
+        finish_timing(ctx);
         return len > out_cap ? fail(PJ_ERR_CAPACITY, "output capacity too small") : PJ_OK;
     }
     P.n = m;
@@ -689,10 +777,9 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
     P.total = ec + 1;
     P.state = ec + 2;
     PJ_HIP(pj_launch_encode_rows(P, format == PJ_FORMAT_PRETTY, ctx->stream));
-    if ((s = mark(ctx))) return s;
-    PJ_HIP(hipMemcpyAsync(ctx->pinned, ec + 1, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    PJ_HIP(pj_launch_publish(ctx->pinned, ec + 1, 1, 0, -1, ctx->stream, mark(ctx)));
     PJ_HIP(hipStreamSynchronize(ctx->stream));
-    if ((s = finish_timing(ctx))) return s;
+    finish_timing(ctx);
     *out_len = ctx->pinned[0];
     if (*out_len > out_cap) return fail(PJ_ERR_CAPACITY, "output capacity too small");
     return PJ_OK;
@@ -1075,7 +1162,6 @@ bool dec_cols_ok(const pj_pet_columns *o) {
 // (~0 when it has none), and no frame check is made.
 pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, DecParams &P, uint64_t *&X,
                       uint64_t *lines_out, uint64_t *cut = nullptr) {
-    pj_status s;
     const uint64_t nblk64 = (len + 63) / 64;
     uint64_t ls_cap = len / 128 + 16;
     for (int attempt = 0; attempt < 2; attempt++) {
@@ -1083,13 +1169,13 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
         // (the newline index's, or the array frame's blocks)
         const uint64_t ga = array ? pj_arr_blocks(nblk64) : 0;
         const uint64_t gidx = std::max((nblk64 + pj_dec_index_block() - 1) / pj_dec_index_block(), ga);
-        // layout (u64 units): header 16 | dummy 32 | array frame scalars 8 |
+        // layout (u64 units): header 16 | array frame scalars 8 | dummy 32 |
         //   state_idx gidx | (arrays: block summaries, entry states, per-thread
         //   summaries) | line_start ls_cap
         // header: 0-1 tickets, 2 line count, 3 blank lines, 4-11 totals,
         //         12 lines off the fast path, 13 deferred error-code queue
         //         length, 14 lines for k_dec_long, 15 scan ticket
-        const uint64_t o_dummy = 16, o_arr = 48, o_sidx = 56;
+        const uint64_t o_arr = 16, o_dummy = 24, o_sidx = 56;
         const uint64_t o_bsum = o_sidx + gidx, o_bpre = o_bsum + (ga * sizeof(FS) + 7) / 8;
         const uint64_t o_tsum = o_bpre + ga, ta = array ? pj_arr_threads(nblk64) : 0;
         const uint64_t o_ls = o_tsum + (ta * sizeof(FS) + 7) / 8;
@@ -1110,6 +1196,8 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
         P.empty_count = reinterpret_cast<unsigned long long *>(X + 3);
         P.array_doc = array ? 1 : 0;
         P.arr = X + o_arr;
+        P.head = X;
+        P.host = ctx->pinned;
         P.arr_bsum = reinterpret_cast<FS *>(X + o_bsum);
         P.arr_bpre = X + o_bpre;
         P.arr_tsum = reinterpret_cast<FS *>(X + o_tsum);
@@ -1119,22 +1207,25 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
         P.spin_limit = spin_limit();
         for (;;) {
             ctx->n_ev = 0;
-            if ((s = mark(ctx))) return s;
-            PJ_HIP(pj_launch_fill_u64(X, 16, 0, ctx->stream));
-            PJ_HIP(pj_launch_fill_u64(X + o_sidx, gidx, 0, ctx->stream));
+            FillRanges R{};
+            R.add(X, 16, 0);
+            R.add(X + o_sidx, gidx, 0);
             if (array) {
-                PJ_HIP(pj_launch_fill_u64(X + o_arr, 8, 0, ctx->stream));
-                PJ_HIP(pj_launch_fill_u64(X + o_arr, 1, ~0ull, ctx->stream));      // first non-whitespace
-                PJ_HIP(pj_launch_fill_u64(X + o_arr + 2, 1, ~0ull, ctx->stream));  // the close
+                R.add(X + o_arr, 1, ~0ull);      // first non-whitespace
+                R.add(X + o_arr + 1, 1, 0);
+                R.add(X + o_arr + 2, 1, ~0ull);  // the close
+                R.add(X + o_arr + 3, 5, 0);
             }
-            if ((s = mark(ctx))) return s;
+            PJ_HIP(pj_launch_fill_ranges(R, ctx->stream, mark(ctx)));
+            P.stamp = mark(ctx);
+            P.stamp2 = mark(ctx);
+            if (!nblk64) *P.stamp = 0;           // no index kernel runs
             if (array) PJ_HIP(pj_launch_arr_frame(P, ctx->stream));
             else if (nblk64) PJ_HIP(pj_launch_dec_index(P, ctx->stream));
-            if ((s = mark(ctx))) return s;
-            PJ_HIP(hipMemcpyAsync(ctx->pinned, X, 3 * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-            if (array) PJ_HIP(hipMemcpyAsync(ctx->pinned + 16, X + o_arr, 8 * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                                             ctx->stream));
+            // (k_arr_fin copies the header and the frame's scalars itself)
+            if (!array) PJ_HIP(pj_launch_publish(ctx->pinned, X, 3, 0, -1, ctx->stream, P.stamp2));
             PJ_HIP(hipStreamSynchronize(ctx->stream));
+            if (!nblk64) *P.stamp = *P.stamp2;
             if (array || !P.order_by_id || ctx->pinned[0] == 0) break;
             P.order_by_id = 0;
         }
@@ -1152,7 +1243,7 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
             return PJ_OK;
         }
         if (array && ctx->pinned[16 + 4] == 0) {
-            (void)finish_timing(ctx);
+            finish_timing(ctx);
             return fail(PJ_ERR_SYNTAX, "not a JSON array: '[', the top-level commas or the closing ']' are malformed");
         }
         const uint64_t lines = ctx->pinned[2];
@@ -1220,6 +1311,7 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     const uint64_t w_lpos = (9 * lines + 1) / 2;
     const uint64_t w_split = split ? lines + w_lpos + 2 + gp : 0;
     PJ_HIP(ctx->scan.ensure((w_state + lines + 8 + w_split) * 8));
+    ctx->scan_zero = 0;
     uint64_t *SB = static_cast<uint64_t *>(ctx->scan.p);
     P.state_parse = SB;
     P.bagg = SB;
@@ -1236,41 +1328,42 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     P.bm_list = P.long_list + lines + w_lpos + 2;
     P.order_by_id = 1;
     for (;;) {
-        if ((s = mark(ctx))) return s;
+        FillRanges R{};
         if (split) {
-            PJ_HIP(pj_launch_fill_u64(P.bstate, nsb * VLB_WORDS, 0, ctx->stream));
-            PJ_HIP(pj_launch_fill_u64(reinterpret_cast<uint64_t *>(P.bm_count), 2, 0, ctx->stream));
-        }
-        else PJ_HIP(pj_launch_fill_u64(P.state_parse, gp * VLB_WORDS, 0, ctx->stream));
-        PJ_HIP(pj_launch_fill_u64(X + 1, 1, 0, ctx->stream));      // the parse ticket / give-up word
-        PJ_HIP(pj_launch_fill_u64(X + 3, 13, 0, ctx->stream));     // totals and counters
-        if ((s = mark(ctx))) return s;
-        if (lines) {
-            PJ_HIP(pj_launch_dec_parse(P, ctx->stream));
-            if (split) {
-                if ((s = mark(ctx))) return s;
-                PJ_HIP(pj_launch_dec_bscan(P, ctx->stream));
-                if ((s = mark(ctx))) return s;
-                PJ_HIP(pj_launch_dec_write(P, ctx->stream));
-                if ((s = mark(ctx))) return s;
-                PJ_HIP(pj_launch_dec_long(P, ctx->stream));
-            }
-            if ((s = mark(ctx))) return s;
-            PJ_HIP(pj_launch_dec_errcode(P, ctx->stream));
-        } else {
-            // no lines: the offset arrays still start with 0
+            R.add(P.bstate, nsb * VLB_WORDS, 0);
+            R.add(reinterpret_cast<uint64_t *>(P.bm_count), 2, 0);
+        } else R.add(P.state_parse, gp * VLB_WORDS, 0);
+        R.add(X + 1, 1, 0);      // the parse ticket / give-up word
+        R.add(X + 3, 13, 0);     // totals and counters
+        if (!lines) {            // the offset arrays still start with 0
             uint64_t *heads[6] = {out->name_off, out->cat_name_off, out->photo_off, out->tag_off, out->url_off,
                                   out->tag_name_off};
-            for (uint64_t *h : heads) PJ_HIP(pj_launch_fill_u64(h, 1, 0, ctx->stream));
+            R.k = 0;
+            for (uint64_t *h : heads) R.add(h, 1, 0);
+            R.add(X + 3, 13, 0);
         }
-        if ((s = mark(ctx))) return s;
-        PJ_HIP(hipMemcpyAsync(ctx->pinned, X, 13 * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        PJ_HIP(pj_launch_fill_ranges(R, ctx->stream, mark(ctx)));
+        if (lines) {
+            P.stamp = mark(ctx);
+            PJ_HIP(pj_launch_dec_parse(P, ctx->stream));
+            if (split) {
+                P.stamp = mark(ctx);
+                PJ_HIP(pj_launch_dec_bscan(P, ctx->stream));
+                P.stamp = mark(ctx);
+                PJ_HIP(pj_launch_dec_write(P, ctx->stream));
+                P.stamp = mark(ctx);
+                PJ_HIP(pj_launch_dec_long(P, ctx->stream));
+            }
+            P.stamp = mark(ctx);
+            PJ_HIP(pj_launch_dec_errcode(P, ctx->stream));
+        }
+        PJ_HIP(pj_launch_publish(ctx->pinned, X, 13, 0, -1, ctx->stream, mark(ctx)));
         PJ_HIP(hipStreamSynchronize(ctx->stream));
         if (!P.order_by_id || ctx->pinned[1] == 0) break;
         P.order_by_id = 0;
         ctx->n_ev = 0;
     }
-    if ((s = finish_timing(ctx))) return s;
+    finish_timing(ctx);
     const uint64_t *T = ctx->pinned + 4;
     res->n_general = lines ? ctx->pinned[12] : 0;
     res->n_lines = lines;
@@ -1617,7 +1710,7 @@ pj_status decode_host_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_
     for (int k = 0; k < 19; k++) off[k + 1] = off[k] + align256(sz[k] + 8);
     PJ_HIP(ctx->stage_out.ensure(off[19]));
     uint8_t *D = static_cast<uint8_t *>(ctx->stage_out.p);
-    if (len && (s = h2d(ctx, D, in, len))) return s;
+    if ((s = h2d_input(ctx, D, in, len))) return s;
     void *dp[17];
     for (int k = 0; k < 17; k++) dp[k] = D + off[k];
     pj_pet_columns dc = *out;
@@ -1625,7 +1718,10 @@ pj_status decode_host_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_
     uint64_t *del = reinterpret_cast<uint64_t *>(D + off[17]);
     uint8_t *dec = D + off[18];
     s = decode_impl(ctx, D, len, &dc, err_cap ? del : nullptr, err_cap ? dec : nullptr, err_cap, res, array);
-    if (s != PJ_OK && s != PJ_ERR_CAPACITY) return s;
+    if (s != PJ_OK && s != PJ_ERR_CAPACITY) {
+        (void)hipStreamSynchronize(ctx->stream);       // the queued input copy has left its buffer
+        return s;
+    }
     const uint64_t np = std::min(res->n_pets, cp), nu = std::min(res->n_urls, cu), nt = std::min(res->n_tags, ct);
     const uint64_t used[17] = {np * 8, np, np, (np + 1) * 8, std::min(res->name_bytes, out->cap_name_bytes), np * 8,
                                np, (np + 1) * 8, std::min(res->cat_name_bytes, out->cap_cat_name_bytes),
@@ -1634,13 +1730,12 @@ pj_status decode_host_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_
                                std::min(res->tag_name_bytes, out->cap_tag_name_bytes)};
     void *hp[17];
     col_ptrs(out, hp);
-    pj_status t = PJ_OK;
-    for (int k = 0; k < 17; k++)
-        if (used[k] && (t = d2h(ctx, hp[k], dp[k], used[k], nullptr, false))) return t;
     const uint64_t ne = std::min(res->n_errors, err_cap);
-    if (ne && ((t = d2h(ctx, err_line, del, ne * 8, nullptr, false)) || (t = d2h(ctx, err_code, dec, ne, nullptr, false))))
-        return t;
-    if ((t = d2h_wait(ctx))) return t;
+    Piece pc[19];
+    for (int k = 0; k < 17; k++) pc[k] = Piece{hp[k], dp[k], used[k]};
+    pc[17] = Piece{err_line, del, ne * 8};
+    pc[18] = Piece{err_code, dec, ne};
+    if (const pj_status t = d2h_pieces(ctx, pc, 19)) return t;
     out->n_pets = np;
     return s;
 }
@@ -1686,6 +1781,7 @@ extern "C" pj_status pj_encode_model_device(pj_ctx *ctx, int model, const pj_mod
     }
     const uint64_t bt = (uint64_t)pj_encode_model_records(), nblk = (n + bt - 1) / bt;
     PJ_HIP(ctx->scan.ensure((nblk + 2) * sizeof(uint64_t)));
+    ctx->scan_zero = 0;
     uint64_t *sc = static_cast<uint64_t *>(ctx->scan.p);
     ModelEncParams P;
     std::memset(&P, 0, sizeof P);
@@ -1700,14 +1796,12 @@ extern "C" pj_status pj_encode_model_device(pj_ctx *ctx, int model, const pj_mod
     P.ticket = reinterpret_cast<unsigned long long *>(sc);
     P.total = sc + 1;
     P.state = sc + 2;
-    if ((s = mark(ctx))) return s;
-    PJ_HIP(pj_launch_fill_u64(sc, nblk + 2, 0, ctx->stream));
-    if ((s = mark(ctx))) return s;
+    PJ_HIP(pj_launch_fill_u64(sc, nblk + 2, 0, ctx->stream, mark(ctx)));
+    P.stamp = mark(ctx);
     PJ_HIP(pj_launch_encode_model(P, ctx->stream));
-    if ((s = mark(ctx))) return s;
-    PJ_HIP(hipMemcpyAsync(ctx->pinned, sc + 1, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    PJ_HIP(pj_launch_publish(ctx->pinned, sc + 1, 1, 0, -1, ctx->stream, mark(ctx)));
     PJ_HIP(hipStreamSynchronize(ctx->stream));
-    if ((s = finish_timing(ctx))) return s;
+    finish_timing(ctx);
     *out_len = ctx->pinned[0];
     if (*out_len > out_cap) return fail(PJ_ERR_CAPACITY, "output capacity too small");
     return PJ_OK;
@@ -1731,6 +1825,7 @@ extern "C" pj_status pj_decode_model_device(pj_ctx *ctx, int model, const uint8_
     const uint64_t nb = (lines + pj_decode_model_block() - 1) / pj_decode_model_block();
     const uint64_t nchunks = (nb + 1023) / 1024;     // the scan's chunks of 1024 blocks
     PJ_HIP(ctx->scan.ensure((2 * nb * MD_MAXK + nchunks * MD_MAXK + MD_MAXK + 1) * sizeof(uint64_t)));
+    ctx->scan_zero = 0;
     uint64_t *SB = static_cast<uint64_t *>(ctx->scan.p);
     ModelDecParams M;
     std::memset(&M, 0, sizeof M);
@@ -1754,16 +1849,18 @@ extern "C" pj_status pj_decode_model_device(pj_ctx *ctx, int model, const uint8_
         PJ_HIP(ctx->tape.ensure(tw * 8));
         M.tape = static_cast<uint64_t *>(ctx->tape.p);
     }
-    if ((s = mark(ctx))) return s;
-    PJ_HIP(pj_launch_fill_u64(SB, MD_MAXK + 1, 0, ctx->stream));
+    FillRanges R{};
+    R.add(SB, MD_MAXK + 1, 0);
     for (int k = 0; k < model_props(model); k++)    // string offsets start at 0
-        if (model_str(model, k)) PJ_HIP(pj_launch_fill_u64(static_cast<uint64_t *>(out->col[k]), 1, 0, ctx->stream));
-    if ((s = mark(ctx))) return s;
+        if (model_str(model, k)) R.add(static_cast<uint64_t *>(out->col[k]), 1, 0);
+    PJ_HIP(pj_launch_fill_ranges(R, ctx->stream, mark(ctx)));
+    M.stamp = mark(ctx);
     PJ_HIP(pj_launch_decode_model(M, model, ctx->stream));
-    if ((s = mark(ctx))) return s;
-    PJ_HIP(hipMemcpyAsync(ctx->pinned, SB, (MD_MAXK + 1) * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    uint64_t *t1 = mark(ctx);
+    PJ_HIP(pj_launch_publish(ctx->pinned, SB, MD_MAXK + 1, 0, -1, ctx->stream, t1));
     PJ_HIP(hipStreamSynchronize(ctx->stream));
-    if ((s = finish_timing(ctx))) return s;
+    if (!nb) *M.stamp = *t1;                 // no record, no kernel
+    finish_timing(ctx);
     const uint64_t *T = ctx->pinned;
     for (int k = 0; k < PJ_MODEL_MAX_PROPS; k++) out->n_bytes[k] = 0;
     if (array && lines && T[MD_MAXK]) {
@@ -1894,29 +1991,31 @@ extern "C" pj_status pj_decode_model_host(pj_ctx *ctx, int model, const uint8_t 
         dc.col[k] = ob + o_col[k];
         if (model_str(model, k)) dc.bytes[k] = ob + o_bytes[k];
     }
-    if (len && (s = h2d(ctx, D, in, len))) return s;
+    if ((s = h2d_input(ctx, D, in, len))) return s;
     uint64_t *del = reinterpret_cast<uint64_t *>(ob + o_el);
     uint8_t *dec = ob + o_ec;
     s = pj_decode_model_device(ctx, model, D, len, array, &dc, err_cap ? del : nullptr, err_cap ? dec : nullptr,
                                err_cap, res);
-    if (s != PJ_OK && s != PJ_ERR_CAPACITY) return s;
+    if (s != PJ_OK && s != PJ_ERR_CAPACITY) {
+        (void)hipStreamSynchronize(ctx->stream);       // the queued input copy has left its buffer
+        return s;
+    }
     const pj_status ds = s;
     // what was written: the rows that fit, their string bytes, the errors listed
     const uint64_t rows = dc.n;
     out->n = rows;
     for (int k = 0; k < PJ_MODEL_MAX_PROPS; k++) out->n_bytes[k] = dc.n_bytes[k];
-    pj_status t;
-    if ((t = d2h(ctx, out->present, dc.present, rows, nullptr, false))) return t;
+    Piece pc[3 + 2 * PJ_MODEL_MAX_PROPS];
+    int np = 0;
+    pc[np++] = Piece{out->present, dc.present, rows};
     for (int k = 0; k < model_props(model); k++) {
-        if (model_str(model, k)) {
-            if ((t = d2h(ctx, out->col[k], dc.col[k], (rows + 1) * 8, nullptr, false))) return t;
-            const uint64_t nb = std::min(dc.n_bytes[k], out->cap_bytes[k]);
-            if ((t = d2h(ctx, out->bytes[k], dc.bytes[k], nb, nullptr, false))) return t;
-        } else if ((t = d2h(ctx, out->col[k], dc.col[k], model_col_bytes(model, k, rows), nullptr, false))) return t;
+        pc[np++] = Piece{out->col[k], dc.col[k], model_col_bytes(model, k, rows)};
+        if (model_str(model, k))
+            pc[np++] = Piece{out->bytes[k], dc.bytes[k], std::min(dc.n_bytes[k], out->cap_bytes[k])};
     }
     const uint64_t ne = std::min(res->n_errors, err_cap);
-    if (ne && ((t = d2h(ctx, err_line, del, ne * 8, nullptr, false)) || (t = d2h(ctx, err_code, dec, ne, nullptr, false))))
-        return t;
-    if ((t = d2h_wait(ctx))) return t;
+    pc[np++] = Piece{err_line, del, ne * 8};
+    pc[np++] = Piece{err_code, dec, ne};
+    if (const pj_status t = d2h_pieces(ctx, pc, np)) return t;
     return ds == PJ_OK ? PJ_OK : fail(PJ_ERR_CAPACITY, "capacity too small (sizes needed are in the result)");
 }

@@ -25,6 +25,8 @@
 // UTF8StreamJsonParser, comments rejected per reference application.yml:23-28;
 // serde bean binding of the petstore Pet, petstore.json:858-936) are the ones
 // restated by the CPU checker in oracle/pj_oracle.c.
+#include <algorithm>
+
 #include "pj_device.h"
 #include "pj_kernels.h"
 
@@ -151,6 +153,7 @@ __device__ __forceinline__ uint64_t block_excl_scan_idx(uint64_t v, uint64_t *sh
 // look-back of newline counts -> line starts.
 template <int BT, int R>
 __global__ __launch_bounds__(BT) void k_dec_lines(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ uint32_t sh_scan[R * BT / 64];
     __shared__ uint64_t sh_blk, sh_pre;
     const uint32_t t = threadIdx.x;
@@ -349,6 +352,7 @@ __device__ __forceinline__ FS block_fs_scan(FS v, FS *sh) {
 // the loads of ARR_U words, one 128-byte line, in flight together).
 template <int BT, int R, int ARR_U = (R > 1 ? 2 : 1)>
 __global__ __launch_bounds__(BT) void k_arr_sum(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ FS sh[BT];
     const uint32_t t = threadIdx.x;
     const uint64_t b = blockIdx.x, w0 = (b * BT + t) * R;
@@ -366,6 +370,7 @@ __global__ __launch_bounds__(BT) void k_arr_sum(DecParams P) {
     }
     acc = block_fs_scan<BT>(acc, sh);
     if (t == BT - 1) P.arr_bsum[b] = acc;
+    if (gridDim.x == 1 && t == 0) P.arr_bpre[0] = 0;   // (no k_arr_scan: one block, entered at the document's start)
     // the thread's exclusive prefix in the block, for k_arr_frame
     P.arr_tsum[b * BT + t] = t ? sh[t - 1] : fs_id();
 }
@@ -488,20 +493,22 @@ __global__ __launch_bounds__(BT) void k_arr_frame(DecParams P) {
 // The frame's verdict (one thread): the first non-whitespace byte is '[',
 // the close is a ']' after it and nothing but whitespace follows.  Then
 // element 0 starts after the '[' and the last one ends at the ']'.
-__global__ void k_arr_fin(DecParams P) {
-    const uint64_t first = P.arr[0], lastp1 = P.arr[1], close = P.arr[2], nsep = P.arr[3];
-    const bool ok = first != ~0ull && P.in[first] == '[' && close != ~0ull && close > first && P.in[close] == ']' &&
-                    lastp1 == close + 1;
-    P.arr[4] = ok ? 1 : 0;
-    if (!ok) {
-        *P.n_lines = 0;
-        return;
+// The header words and the frame's scalars (24 words) then go to the host.
+__global__ __launch_bounds__(64) void k_arr_fin(DecParams P) {
+    stamp_start(P.stamp2);
+    if (threadIdx.x == 0) {
+        const uint64_t first = P.arr[0], lastp1 = P.arr[1], close = P.arr[2], nsep = P.arr[3];
+        const bool ok = first != ~0ull && P.in[first] == '[' && close != ~0ull && close > first &&
+                        P.in[close] == ']' && lastp1 == close + 1;
+        P.arr[4] = ok ? 1 : 0;
+        if (ok && nsep + 1 < P.ls_cap) {
+            P.line_start[0] = first + 1;
+            P.line_start[nsep + 1] = close + 1;
+        }
+        *P.n_lines = ok ? nsep + 1 : 0;
     }
-    if (nsep + 1 < P.ls_cap) {
-        P.line_start[0] = first + 1;
-        P.line_start[nsep + 1] = close + 1;
-    }
-    *P.n_lines = nsep + 1;
+    __syncthreads();
+    if (threadIdx.x < 24) P.host[threadIdx.x] = P.head[threadIdx.x];
 }
 
 // =========================================================== stage 2
@@ -2852,6 +2859,7 @@ __device__ __forceinline__ void dec_block(DecParams &P, const uint64_t b) {
 
 template <int BT, int TILE, int LONG, int LPB = BT, bool TAPE = false, bool BM = true>
 __global__ __launch_bounds__(BT, BM ? 2 : 3) void k_dec_block(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ uint64_t sh_blk;
     if (threadIdx.x == 0) sh_blk = P.order_by_id ? (uint64_t)blockIdx.x : atomicAdd(&P.tickets[1], 1ull);
     __syncthreads();
@@ -2987,6 +2995,7 @@ __device__ __forceinline__ bool dec_room(const DecParams &P) {
 // each line block's first offsets, totals the call's sums.
 template <int BT>
 __global__ __launch_bounds__(BT) void k_dec_bscan(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ uint64_t sh_scan[BT / 64];
     __shared__ uint64_t sh_sb, sh_pre[PJ_DEC_NCNT];
     const uint32_t t = threadIdx.x;
@@ -3029,6 +3038,7 @@ __global__ __launch_bounds__(BT) void k_dec_bscan(DecParams P) {
 // whole wave or the general parser are left to k_dec_long.
 template <int BT, int TILE, int LPB, int LONG>
 __global__ __launch_bounds__(BT, 2) void k_dec_write(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t sh_ls[LPB + 1];
     __shared__ uint16_t sh_sub[LPB + 1];
@@ -3096,6 +3106,7 @@ __global__ __launch_bounds__(BT, 2) void k_dec_write(DecParams P) {
 // Lines of the general parser are read again from the input by one thread.
 template <int TILE, int LPB>
 __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
     __shared__ uint64_t badm[TILE / 64 + 1];
@@ -3174,6 +3185,7 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
 // tile goes through the byte-by-byte parser from global memory.
 template <int BT, int TILE>
 __global__ __launch_bounds__(BT) void k_dec_errcode(DecParams P) {
+    stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
     __shared__ uint64_t badm[TILE / 64 + 1];
@@ -3307,16 +3319,16 @@ hipError_t pj_launch_arr_frame(const DecParams &P, hipStream_t st) {
     if (g) {                                        // an empty document has no frame: the verdict says so
         hipLaunchKernelGGL((small ? pj::k_arr_sum<ARR_BT, 1> : pj::k_arr_sum<ARR_BT, ARR_R>), dim3((unsigned)g),
                            dim3(ARR_BT), 0, st, P);
-        hipLaunchKernelGGL((pj::k_arr_scan<1024>), dim3(1), dim3(1024), 0, st, P, g);
+        if (g > 1) hipLaunchKernelGGL((pj::k_arr_scan<1024>), dim3(1), dim3(1024), 0, st, P, g);
         hipLaunchKernelGGL((small ? pj::k_arr_frame<ARR_BT, 1> : pj::k_arr_frame<ARR_BT, ARR_R>), dim3((unsigned)g),
                            dim3(ARR_BT), 0, st, P);
     }
-    hipLaunchKernelGGL(pj::k_arr_fin, dim3(1), dim3(1), 0, st, P);
+    hipLaunchKernelGGL(pj::k_arr_fin, dim3(1), dim3(64), 0, st, P);
     return hipGetLastError();
 }
 
 hipError_t pj_launch_dec_errcode(const DecParams &P, hipStream_t st) {
-    hipLaunchKernelGGL((pj::k_dec_errcode<64, DEC_TILE>), dim3(8192), dim3(64), 0, st, P);
+    hipLaunchKernelGGL((pj::k_dec_errcode<64, DEC_TILE>), dim3((unsigned)std::min<uint64_t>(8192, P.lines)), dim3(64), 0, st, P);
     return hipGetLastError();
 }
 
@@ -3336,7 +3348,8 @@ hipError_t pj_launch_dec_write(const DecParams &P, hipStream_t st) {
 }
 
 hipError_t pj_launch_dec_long(const DecParams &P, hipStream_t st) {
-    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, DEC_LPB>), dim3(1024), dim3(64), 0, st, P);
+    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, DEC_LPB>), dim3((unsigned)std::min<uint64_t>(1024, P.lines)), dim3(64), 0,
+                       st, P);
     return hipGetLastError();
 }
 
@@ -3347,7 +3360,8 @@ hipError_t pj_launch_dec_parse(const DecParams &P, hipStream_t st) {
         // lines it deferred, then its offsets corrected for them
         hipLaunchKernelGGL((pj::k_dec_block<DEC_LINE_BT, DEC_FTILE, DEC_LONG, DEC_LPB, true, false>), dim3((unsigned)g),
                            dim3(DEC_LINE_BT), 0, st, P);
-        hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_TILE>), dim3(1024), dim3(64), 0, st, P);
+        hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_TILE>), dim3((unsigned)std::min<uint64_t>(1024, P.lines)), dim3(64), 0,
+                           st, P);
         hipLaunchKernelGGL((pj::k_dec_fixup<DEC_LINE_BT, DEC_LPB>), dim3((unsigned)(g < 1024 ? g : 1024)),
                            dim3(DEC_LINE_BT), 0, st, P);
     } else

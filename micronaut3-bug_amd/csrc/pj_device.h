@@ -127,6 +127,14 @@ __device__ __forceinline__ void block_excl_scan_n(const uint32_t *v, uint32_t *e
     __syncthreads();
 }
 
+// The wall clock at the start of a launch (its first workgroup), for the call's
+// timings: stamps into pinned memory cost a kernel one store, an event between
+// two kernels about 5 us of the stream's time.
+__device__ __forceinline__ void stamp_start(uint64_t *stamp) {
+    if (stamp && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(stamp, (uint64_t)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ----------------------------------------------------------- look-back
 // One 64-bit word per logical block: bits 63:62 = state, 61:0 = value.
 constexpr uint64_t LB_AGG = 1ull << 62;

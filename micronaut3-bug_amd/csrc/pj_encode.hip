@@ -1412,6 +1412,7 @@ __device__ __forceinline__ void enc_prefetch(const EncParams &P, const Geo &g, R
 // skewed record does not hold its workgroup for long.
 template <bool NESTED, int BT, int R, int TILE, int INCAP, int UCAP, int GCAP, int WPE = 1, bool PRETTY = false>
 __global__ __launch_bounds__(BT, WPE) void k_encode(EncParams P) {
+    stamp_start(P.stamp);
     static_assert(!PRETTY || NESTED, "pretty output through the tile path: nested layout only");
     constexpr int UA = NESTED ? UCAP : 1, GA = NESTED ? GCAP : 1, RA = NESTED ? R : 1;
     // flat records write the tile with aligned stores only; nested ones,
@@ -1880,6 +1881,7 @@ __global__ __launch_bounds__(BT, WPE) void k_encode(EncParams P) {
 // first round (records, items, chunks) is issued before any is used.
 template <int BT, int R, int K, int UN>
 __global__ __launch_bounds__(BT) void k_enc_measure(EncParams P) {
+    stamp_start(P.stamp);
     constexpr int RG = R * K, NW = BT / 64;
     static_assert(RG <= BT, "one record per thread");
     // block boundaries j = 0..K: url item, tag item, then the first byte of
@@ -2072,6 +2074,7 @@ __global__ __launch_bounds__(BT) void k_enc_measure(EncParams P) {
 // capacity are not written; the last block stores the total.
 template <int BT, bool PRETTY>
 __global__ __launch_bounds__(BT) void k_encode_rows(EncParams P) {
+    stamp_start(P.stamp);
     __shared__ uint64_t sh_scan[BT / 64 + 2];
     __shared__ uint64_t sh_b, sh_base;
     const ColSrc XG{P.c.name_bytes, P.c.cat_name_bytes, P.c.url_bytes, P.c.tag_name_bytes, 0, 0, 0, 0};
@@ -2115,6 +2118,7 @@ __global__ __launch_bounds__(BT) void k_encode_rows(EncParams P) {
 // block stores the count.
 template <int BT, int R>
 __global__ __launch_bounds__(BT) void k_select_status(EncParams P, uint32_t mask, uint64_t *sel) {
+    stamp_start(P.stamp);
     __shared__ uint64_t sh_scan[BT / 64 + 2];
     __shared__ uint64_t sh_b, sh_base;
     const uint32_t t = threadIdx.x;
@@ -2266,6 +2270,7 @@ __device__ __forceinline__ void m_rec(S &s, const ModelEncParams &P, uint64_t i,
 // the values again and stored 32-byte sectors from each thread.
 template <int MODEL, bool PRETTY, int BT, int TILE>
 __global__ __launch_bounds__(BT, 4) void k_encode_model(ModelEncParams P) {
+    stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 32];    // tile_copy_out reads 32 bytes past
     __shared__ uint64_t sh_scan[BT / 64 + 2];
     __shared__ uint64_t sh_b, sh_base, sh_end;
@@ -2334,9 +2339,47 @@ __global__ void k_add_u64(uint64_t *p, uint64_t n, uint64_t v) {
     if (i < n) p[i] += v;
 }
 
-__global__ void k_fill_u64(uint64_t *p, uint64_t n, uint64_t v) {
+__global__ void k_fill_u64(uint64_t *p, uint64_t n, uint64_t v, uint64_t *stamp) {
+    stamp_start(stamp);
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+// Block blockIdx.x of the ranges' blocks of 256 words, laid end to end.
+__global__ __launch_bounds__(256) void k_fill_ranges(FillRanges R, uint64_t *stamp) {
+    stamp_start(stamp);
+    uint64_t b = blockIdx.x;
+    for (int k = 0; k < R.k; k++) {
+        const uint64_t g = (R.n[k] + 255) / 256;
+        if (b < g) {
+            const uint64_t i = b * 256 + threadIdx.x;
+            if (i < R.n[k]) R.p[k][i] = R.v[k];
+            return;
+        }
+        b -= g;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_publish(uint64_t *host, uint64_t *src, int n, uint64_t zero, int keep,
+                                                 uint64_t *stamp) {
+    stamp_start(stamp);
+    for (uint64_t i = threadIdx.x; i < (uint64_t)n || i < zero; i += 256) {
+        if (i < (uint64_t)n) host[i] = src[i];
+        if (i < zero && (int64_t)i != keep) src[i] = 0;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_copy_pieces(CopyPieces C) {
+    uint64_t b = blockIdx.x;
+    for (int k = 0; k < C.k; k++) {
+        const uint64_t m = (C.n[k] + 15) / 16, g = (m + 255) / 256;
+        if (b < g) {
+            const uint64_t i = b * 256 + threadIdx.x;
+            if (i < m) reinterpret_cast<uint4 *>(C.dst[k])[i] = reinterpret_cast<const uint4 *>(C.src[k])[i];
+            return;
+        }
+        b -= g;
+    }
 }
 
 __global__ void k_put_bytes(uint8_t *out, uint32_t w, int k) {
@@ -2353,10 +2396,32 @@ hipError_t pj_launch_add_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st
     return hipGetLastError();
 }
 
-hipError_t pj_launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st) {
+hipError_t pj_launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st, uint64_t *stamp) {
     if (n == 0) return hipSuccess;
     uint64_t g = (n + 255) / 256;
-    hipLaunchKernelGGL(pj::k_fill_u64, dim3((unsigned)g), dim3(256), 0, st, p, n, v);
+    hipLaunchKernelGGL(pj::k_fill_u64, dim3((unsigned)g), dim3(256), 0, st, p, n, v, stamp);
+    return hipGetLastError();
+}
+
+hipError_t pj_launch_fill_ranges(const FillRanges &R, hipStream_t st, uint64_t *stamp) {
+    uint64_t g = 0;
+    for (int k = 0; k < R.k; k++) g += (R.n[k] + 255) / 256;
+    if (!g) return hipSuccess;
+    hipLaunchKernelGGL(pj::k_fill_ranges, dim3((unsigned)g), dim3(256), 0, st, R, stamp);
+    return hipGetLastError();
+}
+
+hipError_t pj_launch_publish(uint64_t *host, uint64_t *src, int n, uint64_t zero, int keep, hipStream_t st,
+                             uint64_t *stamp) {
+    hipLaunchKernelGGL(pj::k_publish, dim3(1), dim3(256), 0, st, host, src, n, zero, keep, stamp);
+    return hipGetLastError();
+}
+
+hipError_t pj_launch_copy_pieces(const CopyPieces &C, hipStream_t st) {
+    uint64_t g = 0;
+    for (int k = 0; k < C.k; k++) g += ((C.n[k] + 15) / 16 + 255) / 256;
+    if (!g) return hipSuccess;
+    hipLaunchKernelGGL(pj::k_copy_pieces, dim3((unsigned)g), dim3(256), 0, st, C);
     return hipGetLastError();
 }
 

@@ -30,6 +30,7 @@ struct EncParams {
     // nested writer: large records are listed (record, output offset) for
     // k_enc_big to write after the pass; with big_cap 0, or once the list
     // is full, the pass writes them itself
+    uint64_t *stamp;           // start-of-launch clock stamp, or null
     unsigned long long *big_count;  // zeroed
     uint64_t *big_list;
     uint64_t big_cap;
@@ -51,6 +52,7 @@ struct ModelEncParams {
     uint64_t *state;           // look-back words, one per block (zeroed)
     unsigned long long *ticket;// block ticket (zeroed)
     uint64_t *total;           // encoded size (written by the last block)
+    uint64_t *stamp;           // start-of-launch clock stamp, or null
 };
 
 // Order / User decode (pj_decode_model_device), after the record index:
@@ -72,6 +74,7 @@ struct ModelDecParams {
     uint64_t nblocks;
     uint64_t *tape;            // what the counting pass read of each record, for the writer
                                // (word k of record l at tape[k * lines + l]), or null
+    uint64_t *stamp;           // start-of-launch clock stamp, or null
 };
 
 // What the decode counting kernels learn about each line, read back by the
@@ -145,12 +148,43 @@ struct DecParams {
     // in ticket order
     int order_by_id;
     uint64_t spin_limit;
+    uint64_t *host;            // array frame: pinned words that k_arr_fin copies the header and the frame's scalars to
+    const uint64_t *head;      // (from here)
+    uint64_t *stamp, *stamp2;  // start-of-launch clock stamps (stamp2: k_arr_fin's), or null
 };
 
 // counters carried through the parse-stage scan
 enum { C_PETS = 0, C_NAMEB, C_CATB, C_URLS, C_URLB, C_TAGS, C_TAGB, C_ERRS, PJ_DEC_NCNT };
 
-hipError_t pj_launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st);
+hipError_t pj_launch_fill_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st, uint64_t *stamp = nullptr);
+// Up to eight ranges of words filled by one launch.
+struct FillRanges {
+    uint64_t *p[8];
+    uint64_t n[8], v[8];
+    int k;
+    void add(uint64_t *q, uint64_t count, uint64_t value) {
+        p[k] = q;
+        n[k] = count;
+        v[k++] = value;
+    }
+};
+hipError_t pj_launch_fill_ranges(const FillRanges &R, hipStream_t st, uint64_t *stamp = nullptr);
+// n words from device memory to pinned host memory by one small launch (a
+// copy call of a few words costs the host more than a kernel); the first
+// `zero` words of src are then cleared, but for src[keep] (keep < 0: none).
+hipError_t pj_launch_publish(uint64_t *host, uint64_t *src, int n, uint64_t zero, int keep, hipStream_t st,
+                             uint64_t *stamp = nullptr);
+// Up to 20 pieces gathered into dst (or scattered from it) by one launch, 16
+// bytes per access: sources and destinations are 16-byte aligned and hold
+// each piece's size rounded up to 16 bytes.  Either side may be pinned host
+// memory.
+struct CopyPieces {
+    uint8_t *dst[20];
+    const uint8_t *src[20];
+    uint64_t n[20];
+    int k;
+};
+hipError_t pj_launch_copy_pieces(const CopyPieces &C, hipStream_t st);
 hipError_t pj_launch_add_u64(uint64_t *p, uint64_t n, uint64_t v, hipStream_t st);   // p[0, n) += v
 hipError_t pj_launch_encode(const EncParams &P, bool nested, bool wide, hipStream_t st);
 hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t st);

@@ -843,6 +843,7 @@ template <int MODEL> constexpr bool m_counter(int k) {
 // Five workgroups fit a CU's LDS (32 KiB each).
 template <int MODEL, int BT, int TILE>
 __global__ __launch_bounds__(BT) void k_mdec_count(ModelDecParams P) {
+    stamp_start(P.stamp);
     constexpr int NW = BT / 64;
     __shared__ uint64_t sh[NW][MD_MAXK];
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + M_PAD];

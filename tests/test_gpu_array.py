@@ -163,3 +163,30 @@ def test_array_million_records(codec):
     assert res.n_lines == n and res.n_errors == 0 and res.n_pets == n
     for k in pj.COLS:
         assert torch.equal(dev[k].contiguous().view(torch.uint8), dcols[k].contiguous().view(torch.uint8)), k
+
+
+@pytest.mark.parametrize("size", [16 * 2**20 - 64, 16 * 2**20, 16 * 2**20 + 1, 16 * 2**20 + 64, 17_500_003])
+def test_array_frame_words_per_thread(codec, size):
+    """Documents of up to 16 MiB give each thread of the frame kernels one
+    64-byte word, longer ones eight: sizes on both sides of the line, with
+    separators, brackets, escaped quotes and backslash runs inside strings
+    laid across the edges of words, thread runs (512 bytes) and blocks (16
+    and 128 KiB)."""
+    hairy = [b'{"name":"a,b]}\\\\\\"[{","photoUrls":["\\\\","x\\\\\\\\"],"id":%d}', b'{"name":"%d","photoUrls":[]}',
+             b' \n{ "name" : "\\\\\\\\\\"" , "photoUrls" : [ "],[" ] , "x" : [[{"y":"}"},%d],{}] }\t']
+    elems, used = [], 1
+    edges = [e for e in sorted(k * step for step, n in ((16384, 9), (131072, 130), (512, 5), (64, 9)) for k in range(1, n))
+             if e < size - 2000]
+    for i, edge in enumerate(edges + [size - 400]):
+        pad = edge - used - 2 - i % 24                      # the next hairy element starts just before the edge
+        if pad > 60:
+            elems.append(b'{"name":"' + b"p" * (pad - 27) + b'","photoUrls":[]}')
+            used += pad + 1
+        h = hairy[i % 3] % i
+        elems.append(h)
+        used += len(h) + 1
+    doc = b"[" + b",".join(elems)
+    doc += b" " * (size - 1 - len(doc)) + b"]"
+    assert len(doc) == size
+    ref = orc.decode_array(doc)
+    assert_same(doc, gpu_array(codec, doc), ref)

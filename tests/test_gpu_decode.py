@@ -612,3 +612,24 @@ def test_config4_full_size_with_corruption(codec):
         assert torch.equal(got, v.contiguous().view(torch.uint8)), k
     del dcols, dev, exp
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("shift", [0, 5])
+def test_decode_long_line_bitmaps_at_word_and_round_edges(codec, shift):
+    """A long line's bitmaps are built 64 words (4 KiB) per round, a word per
+    lane; what a word owes its successor crosses lanes and rounds.  Backslash
+    runs, multi-byte characters (whole, cut and stray) and raw controls are
+    laid across word and round edges, against the oracle."""
+    marks = [b"\\\\" * 3 + b'\\"', b"\\\\" * 40, "é".encode(), "€".encode(), "\U0001f600".encode(), b"\xe2\x82",
+             b"\xf0\x9f\x98", b"\x80", b"\x01", b"\\u00e9", b"\\ud83d\\ude00", b"\\", b"\xc3"]
+    lines = []
+    for m in marks:
+        for edge in (4096, 8192, 64 * 70):
+            for back in (1, 2, 3, len(m) // 2 + 1, len(m)):
+                head = b'{"id":7,"name":"'
+                body = b"n" * (edge - len(head) - back) + m + b"z" * 900
+                lines.append(head + body + b'","photoUrls":["u"],"tags":[{"id":1,"name":"t"}]}')
+                # the same two properties earlier in the line: the line starts off the word edges
+                lines.append(b'{"id":7,"category":{"id":1,"name":"c"},"name":"' + body[31:] + b'","photoUrls":[]}')
+    data = b"\n".join(lines) + b"\n"
+    assert_same(gpu_decode(codec, data, shift=shift), orc.decode(data))

@@ -572,3 +572,49 @@ def test_encode_long_names_written_by_waves(codec, esc_rate):
     cols = _with_names(pj.generate(3, 3_000), lens, rng, esc_rate)
     for fmt in (pj.FORMAT_ARRAY, pj.FORMAT_NDJSON):
         assert gpu_encode(codec, cols, fmt) == orc.encode(cols, fmt), fmt
+
+
+def test_encode_scratch_left_clear_between_calls(codec):
+    """An encode clears the scratch words of its pass as its results go out,
+    so that the next one need not: calls of every kind that write the same
+    scratch in between (flat, nested, pretty, sizes, selections, decodes,
+    fixed scratch, more records than are cleared), and large records that
+    turn up after calls without any, each against the oracle."""
+    small, flat, skew, many = pj.generate(3, 500), pj.generate(2, 700), pj.generate(5, 400, seed=3), pj.generate(2, 600_000)
+    assert np.diff(skew["name_off"].astype(np.int64)).max() > 512      # large records
+    dev = {id(c): c.to_device() for c in (small, flat, skew, many)}
+    users = pj.generate_model(pj.MODEL_USER, 300, seed=2)
+    ref = {(id(c), f): orc.encode(c, f) for c in (small, flat, skew, many) for f in (pj.FORMAT_ARRAY, pj.FORMAT_PRETTY)}
+    codec.set_options()
+
+    def enc(c, f=pj.FORMAT_ARRAY):
+        out = torch.empty(len(ref[id(c), f]) + 8, dtype=torch.uint8, device="cuda")
+        assert codec.encode(dev[id(c)], f, out=out).cpu().numpy().tobytes() == ref[id(c), f]
+
+    def noise(k):
+        if k == 0:
+            assert codec.encode_size(dev[id(small)]) == len(ref[id(small), pj.FORMAT_ARRAY])
+        elif k == 1:
+            assert codec.encode_by_status(dev[id(small)], 3)[0].cpu().numpy().tobytes() == orc.encode_by_status(small, 3)[0]
+        elif k == 2:
+            text = torch.frombuffer(bytearray(ref[id(small), pj.FORMAT_ARRAY]), dtype=torch.uint8).cuda()
+            assert codec.decode(text, array=True)[3].n_pets == small.n_pets
+        elif k == 3:
+            assert codec.encode_model(users.to_device()).cpu().numpy().tobytes() == orc.encode_model(users, pj.FORMAT_ARRAY)
+        elif k == 4:
+            out = torch.empty(len(ref[id(flat), pj.FORMAT_ARRAY]), dtype=torch.uint8, device="cuda")
+            codec.encode_noalloc(dev[id(flat)], out)
+        elif k == 5:
+            with pytest.raises(pj.PetJsonError):
+                codec.encode(dev[id(small)], out=torch.empty(100, dtype=torch.uint8, device="cuda"))
+        elif k == 6:
+            enc(many)
+    for k in range(8):
+        for c in (small, flat, skew, small, flat):
+            enc(c)
+            noise(k)
+            enc(c, pj.FORMAT_PRETTY)
+    for _ in range(20):                       # past the calls that expect large records again
+        enc(small)
+    enc(skew)
+    enc(skew)

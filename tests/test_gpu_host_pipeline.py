@@ -275,3 +275,61 @@ def test_host_encode_streamed_in_segments(segment, chunk):
         env["PETJSON_XFER_CHUNK"] = str(chunk)
     r = subprocess.run([sys.executable, "-c", ENC_STREAM], capture_output=True, text=True, env=env, timeout=240)
     assert r.returncode == 0 and "streamed encode ok" in r.stdout, r.stdout[-2000:] + r.stderr[-3000:]
+
+
+SMALL = r"""
+import ctypes as C
+import numpy as np
+import petjson as pj, oracle_py as orc
+codec = pj.Codec(0)
+# column bytes from a few KiB to past 4 MiB (one launch to the bounce buffer
+# below, the copy engine above), pinned outputs past 64 KiB
+for n in (0, 1, 3, 150, 400, 11000, 14000, 16000, 20000):
+    text = np.frombuffer(orc.encode(pj.generate(3, n), pj.FORMAT_NDJSON) + b'{"name":1}\n{"name":"x","photoUrls":[]}', np.uint8)
+    ref, rel, rec, rres = orc.decode(text.tobytes())
+    for pinned in (False, True):
+        mk = pj.host_array if pinned else (lambda k, dt: np.empty(k, dt))
+        caps = {"cap_pets": rres.n_pets, "cap_name_bytes": rres.name_bytes, "cap_cat_name_bytes": rres.cat_name_bytes,
+                "cap_urls": rres.n_urls, "cap_url_bytes": rres.url_bytes, "cap_tags": rres.n_tags,
+                "cap_tag_name_bytes": rres.tag_name_bytes}
+        size = {k: len(ref[k]) for k in pj.COLS}
+        arr = {k: mk(size[k] + 1, pj.DTYPES[k]) for k in pj.COLS}
+        for a in arr.values():
+            a.view(np.uint8)[:] = 0xA5
+        src = mk(text.size, np.uint8)
+        src[:] = text
+        el, ec = mk(4, np.uint64), mk(4, np.uint8)
+        s, res = pj.Columns(0, arr, caps).struct(), pj.DecodeResult()
+        rc = codec.L.pj_decode_host(codec.ctx, src.ctypes.data, src.size, C.byref(s), el.ctypes.data, ec.ctypes.data, 4,
+                                    C.byref(res))
+        assert rc == 0 and res.n_pets == rres.n_pets and res.n_errors == 1, (n, pinned, rc)
+        assert el[0] == rel[0] and ec[0] == rec[0]
+        for k in pj.COLS:
+            assert np.array_equal(arr[k][:size[k]], ref[k]), (n, pinned, k)
+            assert (arr[k][size[k]:].view(np.uint8) == 0xA5).all(), (n, pinned, k)
+for n in (0, 1, 150, 5000, 40000):
+    for model in (pj.MODEL_ORDER, pj.MODEL_USER):
+        text = orc.encode_model(pj.generate_model(model, n, seed=n), pj.FORMAT_NDJSON)
+        rc, ref, rel, rec, rres = orc.decode_model(model, text)
+        got, el, ec, res = codec.decode_model_host(model, text)
+        assert res.n_pets == rres.n_pets == n
+        ref = ref.to_host()
+        assert np.array_equal(got.present, ref.present)
+        for a, b in zip(got.col + got.bytes, ref.col + ref.bytes):
+            assert (a is None and b is None) or np.array_equal(a, b)
+codec.close()
+print("small copies ok")
+"""
+
+
+@pytest.mark.parametrize("chunk", [0, 4096, 100_000])
+def test_host_decode_small_copies(chunk):
+    """Host decodes whose bytes go through the bounce buffers in one launch,
+    and those on the other side of that rule (by size, by pinned memory, by
+    the bounce buffers' own size), against the oracle; nothing is written past
+    a column's end."""
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.join(ROOT, "micronaut3-bug_amd"), os.path.join(ROOT, "tests")]))
+    if chunk:
+        env["PETJSON_XFER_CHUNK"] = str(chunk)
+    r = subprocess.run([sys.executable, "-c", SMALL], capture_output=True, text=True, env=env, timeout=240)
+    assert r.returncode == 0 and "small copies ok" in r.stdout, r.stdout[-2000:] + r.stderr[-3000:]
