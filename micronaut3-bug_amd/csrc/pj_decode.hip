@@ -1172,14 +1172,19 @@ __device__ __forceinline__ uint32_t eq_mask8(uint64_t x, uint32_t c) {
     const uint64_t z = ~(((t & m7) + m7) | t) & 0x8080808080808080ull;
     return (uint32_t)(((z >> 7) * 0x0102040810204080ull) >> 56);
 }
-// The stop byte c at q of a string (not its closing quote): an escape, a
-// UTF-8 lead byte with its continuation bytes, or an error.  Returns the
-// bytes consumed | the bytes they decode to << 8, or 0 for an error.
-__device__ __noinline__ uint32_t str_step(const PJ_LDS uint8_t *s, uint32_t n, uint32_t q, uint32_t c) {
+// The stop byte c at q of a string (not its closing quote), w the 8 bytes
+// there: an escape, a UTF-8 lead byte with its continuation bytes, or an
+// error.  Returns the bytes consumed | the bytes they decode to << 8, or 0
+// for an error.  Only surrogates and malformed \u escapes read the line again.
+// (Inlined: as a call it cost k_dec_block 36 of 770 us, and 92 of 808 with
+// k_dec_measure_long on escape-heavy lines.)
+__device__ __forceinline__ uint32_t str_step(const PJ_LDS uint8_t *s, uint32_t n, uint32_t q, uint32_t c, uint64_t w) {
     if (c == '\\') {
-        const uint64_t w = lds_u64(s + q);
         const uint32_t e = (uint32_t)(w >> 8) & 0xFF;
         if (e == 'u') {
+            const int cu = hex4((uint32_t)(w >> 16));
+            if (cu >= 0 && (cu < 0xD800 || cu > 0xDFFF) && q + 6 <= n)
+                return 6u | ((cu < 0x80 ? 1u : cu < 0x800 ? 2u : 3u) << 8);
             const Esc x = escape_at((const uint8_t *)s, n, q);
             return x.err ? 0u : (x.adv | ((uint32_t)x.k << 8));
         }
@@ -1189,7 +1194,7 @@ __device__ __noinline__ uint32_t str_step(const PJ_LDS uint8_t *s, uint32_t n, u
         const bool ok = e < 128 && (((e < 64 ? LO : HI) >> (e & 63)) & 1) && q + 1 < n;
         return ok ? (2u | (1u << 8)) : 0u;
     }
-    const uint32_t extra = utf8_extra(c, lds_u64(s + q));
+    const uint32_t extra = utf8_extra(c, w);
     return extra ? ((1 + extra) | ((1 + extra) << 8)) : 0u;
 }
 
@@ -1428,7 +1433,7 @@ struct FLineT {
             const uint32_t c = (uint32_t)((m0 ? x0 : x1) >> (8 * (k & 7))) & 0xFF;
             if (c == '"') break;
             // an escape, a UTF-8 sequence or an error: out of line
-            const uint32_t st = str_step((const PJ_LDS uint8_t *)s, n, q, c);
+            const uint32_t st = str_step((const PJ_LDS uint8_t *)s, n, q, c, ld8(q));
             if (!st) {
                 r.err = PJ_REC_STRING;
                 return r;
@@ -1921,11 +1926,10 @@ __device__ __forceinline__ uint64_t tape_str(uint32_t q, const Str &r) {
 // subset of properties their lines hold.
 // Pass 0 (WRITE false) validates and measures into R; pass 1 writes the
 // record at the line's offsets rel[] inside the block's column slices W.
-// With TAPE, pass 0 also records the line's tape at T.
-template <bool WRITE, class FL, bool TAPE = false>
-__device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W, const uint32_t *rel,
-                                     Tape T = Tape{nullptr, 0}) {
-    constexpr bool VAL = WRITE || TAPE;             // integer values are needed
+// (fline_tape is pass 0 with the line's tape.)
+template <bool WRITE, class FL>
+__device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W, const uint32_t *rel) {
+    constexpr bool VAL = WRITE;                     // integer values are needed
     const uint32_t n = F.n;
     if (n == 0) return PJ_REC_EMPTY;
     if (F.at(0) != '{') return PJ_BAIL;
@@ -1955,7 +1959,6 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
         if (e) return e;
         flags |= PJ_PET_HAS_CATEGORY;
         cat_len = (cat_fl & PJ_SUB_HAS_NAME) ? nr.dlen : 0;
-        if (TAPE && (cat_fl & PJ_SUB_HAS_NAME)) T[4] = tape_str(nq, nr);
         if (WRITE && cat_len) F.copy(nq, nr, W->cat_name + rel[C_CATB]);
         FL_SEP();
     }
@@ -1968,7 +1971,6 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
         p = r.end + 1;
         flags |= PJ_PET_HAS_NAME;
         name_len = r.dlen;
-        if (TAPE) T[3] = tape_str(q, r);
         if (WRITE && r.dlen) F.copy(q, r, W->name + rel[C_NAMEB]);
         FL_SEP();
     }
@@ -1988,8 +1990,6 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
                 p = r.end + 1;
                 n_urls++;
                 url_bytes += r.dlen;
-                // url k at word 5 + k (n_urls counts it already)
-                if (TAPE && n_urls <= TAPE_WORDS - 5) T[4 + n_urls] = tape_str(q, r);
                 if (WRITE) {
                     if (r.dlen) F.copy(q, r, W->url + ub);
                     ub += r.dlen;
@@ -2026,11 +2026,6 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
                 const uint32_t tl = (tfl & PJ_SUB_HAS_NAME) ? nr.dlen : 0;
                 n_tags++;
                 tag_bytes += tl;
-                // tag k at words 5 + urls + 2k, + 1 (n_tags counts it already)
-                if (TAPE && n_urls + 2 * n_tags <= TAPE_WORDS - 5) {
-                    T[3 + n_urls + 2 * n_tags] = (uint64_t)tid;
-                    T[4 + n_urls + 2 * n_tags] = (tl ? tape_str(nq, nr) : 0) | ((uint64_t)(tfl & 3) << 49);
-                }
                 if (WRITE) {
                     if (F.lead()) {
                         W->tag_id[g] = tid;
@@ -2071,13 +2066,6 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
     if (!WRITE) {
         R.name_len = name_len; R.cat_len = cat_len; R.n_urls = n_urls; R.url_bytes = url_bytes;
         R.n_tags = n_tags; R.tag_bytes = tag_bytes;
-        if (TAPE) {
-            if (n_urls + 2 * n_tags > TAPE_WORDS - 5) return PJ_TAPE_FULL;
-            T[0] = (uint64_t)id;
-            T[1] = (uint64_t)cat_id;
-            T[2] = (uint64_t)flags | ((uint64_t)status << 8) | ((uint64_t)cat_fl << 16) | ((uint64_t)n_urls << 24) |
-                   ((uint64_t)n_tags << 32);
-        }
     } else if (F.lead()) {
         const uint32_t row = rel[C_PETS];
         W->id[row] = id;
@@ -2094,6 +2082,273 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
 }
 #undef FL_SEP
 #undef FL_UNKNOWN
+
+// ------------------------------------------------- the validating walk
+// What fline<false, FLine, true> does (validate, measure, record the tape),
+// written for the least instructions and the fewest dependent LDS reads per
+// line, as it is the decode's longest kernel (bound by instruction issue and
+// LDS latency at two and a half waves per SIMD):
+//   * an integer is three loads at once for its digits and then its last
+//     sixteen digits and what follows it, again at once: no power-of-ten
+//     loops, no byte reads;
+//   * after a value one round of loads brings the separator and the next
+//     key's 16 bytes; item lists read "," and the next opener together;
+//   * unknown properties are looked for once, when no known key follows,
+//     instead of before each property; `last` keeps the schema order then.
+// The byte after a line is its newline (or the tile's zero padding), which no
+// token accepts, so reads need no bounds but the tile's own padding.
+// 3M lines (823 MB): k_dec_block 928 -> 734 us; 250,000 skewed
+// lines (137 MB, escape-heavy names): 740 -> 480 us.  (The next 16 bytes of a
+// string loaded while these are tested: no change, 772 against 770.)
+
+// m (1..8) digits packed in x, first digit lowest
+__device__ __forceinline__ uint32_t digits8_dot(uint64_t x, uint32_t m) {
+    const uint64_t y = (x - 0x3030303030303030ull) << (8 * (8 - m));
+    const uint32_t a = (uint32_t)y, b = (uint32_t)(y >> 32);
+    const uint32_t a1 = __builtin_amdgcn_udot4(a, 0x0000010Au, 0u, false), a2 = __builtin_amdgcn_udot4(a, 0x010A0000u, 0u, false);
+    const uint32_t b1 = __builtin_amdgcn_udot4(b, 0x0000010Au, 0u, false), b2 = __builtin_amdgcn_udot4(b, 0x010A0000u, 0u, false);
+    return (a1 * 100u + a2) * 10000u + (b1 * 100u + b2);
+}
+// The integer at p: p moves past it, a gets the 8 bytes from there on.
+// 0, PJ_REC_NUMBER or PJ_BAIL, as fnum.
+__device__ __forceinline__ int tnum(const FLine &F, uint32_t &p, int64_t &v, uint64_t &a) {
+    const uint64_t w0 = F.ld8(p), w1 = F.ld8(p + 8), w2 = F.ld8(p + 16);
+    const bool neg = (w0 & 0xFF) == '-';
+    const uint64_t c0 = neg ? (w0 >> 8) | (w1 << 56) : w0, c1 = neg ? (w1 >> 8) | (w2 << 56) : w1, c2 = neg ? w2 >> 8 : w2;
+    const uint64_t n0 = nondigit8(c0), n1 = nondigit8(c1), n2 = nondigit8(c2);
+    const uint32_t k = n0   ? (uint32_t)__builtin_ctzll(n0) >> 3
+                       : n1 ? 8 + ((uint32_t)__builtin_ctzll(n1) >> 3)
+                       : n2 ? 16 + ((uint32_t)__builtin_ctzll(n2) >> 3)
+                            : 24;
+    const uint32_t q = p + neg, e = q + k;
+    a = F.ld8(e);
+    if (k == 0 || ((c0 & 0xFF) == '0' && k > 1)) return PJ_BAIL;     // (leading zero: general rules)
+    const uint32_t nx = (uint32_t)a & 0xFF;
+    if (nx != ',' && nx != '}') return PJ_BAIL;                       // fraction, exponent, space...
+    if (k > 19) return PJ_REC_NUMBER;
+    uint64_t u = digits8_dot(c0, k > 16 ? k - 16 : k > 8 ? k - 8 : k);
+    if (k > 8) {
+        const uint64_t lo = F.ld8(e - 8);
+        if (k > 16) u = u * 100000000ull + digits8_dot(F.ld8(e - 16), 8);
+        u = u * 100000000ull + digits8_dot(lo, 8);
+    }
+    if (u > (1ull << 63) - (neg ? 0u : 1u)) return PJ_REC_NUMBER;     // (below 10^19, so u is exact)
+    v = neg ? (int64_t)(0ull - u) : (int64_t)u;
+    p = e;
+    return 0;
+}
+// The string whose content starts at q (FLine::str_swar, the stop byte's
+// window taken from the bytes already loaded).
+__device__ __forceinline__ Str tstr(const FLine &F, uint32_t q) {
+    Str r{0, 0, 0, false};
+    const uint32_t q0 = q;
+    uint32_t shrink = 0;
+    for (;;) {
+        const uint64_t x0 = F.ld8(q), x1 = F.ld8(q + 8);
+        const uint64_t m0 = str_stop8(x0), m1 = str_stop8(x1);
+        if (!(m0 | m1)) {
+            q += 16;
+            continue;
+        }
+        const uint32_t k = m0 ? (uint32_t)__builtin_ctzll(m0) >> 3 : 8 + ((uint32_t)__builtin_ctzll(m1) >> 3);
+        const uint32_t c = (uint32_t)((m0 ? x0 : x1) >> (8 * (k & 7))) & 0xFF;
+        q += k;
+        if (c == '"') break;
+        const uint32_t st = str_step(F.s, F.n, q, c, F.ld8(q));
+        if (!st) {
+            r.err = PJ_REC_STRING;
+            return r;
+        }
+        const uint32_t adv = st & 0xFF, dk = (st >> 8) & 0xFF;
+        q += adv;
+        shrink += adv - dk;
+        r.esc |= c == '\\';
+    }
+    r.end = q;
+    r.dlen = q - q0 - shrink;
+    return r;
+}
+// A Category / Tag body from p (after its '{'): optional "id":N, optional
+// "name":"S"; p moves to its '}', a gets the 8 bytes from there on.
+__device__ __forceinline__ int tsub(const FLine &F, uint32_t &p, int64_t &id, uint32_t &fl, uint32_t &nq, Str &nr, uint64_t &a) {
+    fl = 0;
+    id = 0;
+    uint64_t k8 = F.ld8(p);
+    a = k8;
+    if ((k8 & KP_ID_MASK) == KP_ID) {
+        p += 5;
+        const int e = tnum(F, p, id, a);
+        if (e) return e;
+        fl = PJ_SUB_HAS_ID;
+        if ((a & 0xFF) == ',') {
+            p++;
+            k8 = F.ld8(p);
+            if (k8 != KP_NAME) return PJ_BAIL;
+        } else k8 = 0;
+    }
+    if (k8 == KP_NAME) {
+        nq = p + 8;
+        nr = tstr(F, nq);
+        if (nr.err) return nr.err;
+        p = nr.end + 1;
+        a = F.ld8(p);
+        fl |= PJ_SUB_HAS_NAME;
+    }
+    return (a & 0xFF) == '}' ? 0 : PJ_BAIL;
+}
+__device__ __forceinline__ int fline_tape(const FLine &F, LineRec &R, const Tape T) {
+    const uint32_t n = F.n;
+    if (n == 0) return PJ_REC_EMPTY;
+    uint32_t p = 1, flags = 0, last = 0;
+    uint64_t k8 = F.ld8(1), k16 = F.ld8(9);
+    if (F.s[0] != '{') return PJ_BAIL;
+    uint8_t status = PJ_STATUS_NULL;
+    int64_t id = 0, cat_id = 0;
+    uint32_t cat_fl = 0, name_len = 0, cat_len = 0, n_urls = 0, url_bytes = 0, n_tags = 0, tag_bytes = 0;
+    bool more = (k8 & 0xFF) != '}';
+// after a value at p: ',' brings the next key, '}' ends the object
+#define T_SEP()                                                        \
+    {                                                                  \
+        const uint32_t c_ = F.s[p];                                    \
+        k8 = F.ld8(p + 1);                                             \
+        k16 = F.ld8(p + 9);                                            \
+        if (c_ == ',') p++;                                            \
+        else if (c_ == '}') more = false;                              \
+        else return PJ_BAIL;                                           \
+    }
+    for (;;) {
+        if (more && last < 1 && (k8 & KP_ID_MASK) == KP_ID) {
+            last = 1;
+            p += 5;
+            uint64_t a;
+            const int e = tnum(F, p, id, a);
+            if (e) return e;
+            flags |= PJ_PET_HAS_ID;
+            T_SEP();
+        }
+        if (more && last < 2 && k8 == KP_CATEGORY && (k16 & 0xFFFFFFFFull) == pack8("y\":{", 4)) {
+            last = 2;
+            p += 12;
+            uint32_t nq = 0;
+            uint64_t a;
+            Str nr{0, 0, 0, false};
+            const int e = tsub(F, p, cat_id, cat_fl, nq, nr, a);
+            if (e) return e;
+            p++;
+            flags |= PJ_PET_HAS_CATEGORY;
+            if (cat_fl & PJ_SUB_HAS_NAME) {
+                cat_len = nr.dlen;
+                T[4] = tape_str(nq, nr);
+            }
+            T_SEP();
+        }
+        if (more && last < 3 && k8 == KP_NAME) {
+            last = 3;
+            const uint32_t q = p + 8;
+            const Str r = tstr(F, q);
+            if (r.err) return r.err;
+            p = r.end + 1;
+            flags |= PJ_PET_HAS_NAME;
+            name_len = r.dlen;
+            T[3] = tape_str(q, r);
+            T_SEP();
+        }
+        if (more && last < 4 && k8 == KP_PHOTO && (k16 & 0xFFFFFFFFFFull) == pack8("ls\":[", 5)) {
+            last = 4;
+            flags |= PJ_PET_HAS_PHOTOURLS;
+            uint32_t c = (uint32_t)(k16 >> 40) & 0xFF;            // the byte after '['
+            p += 14;                                              // past it
+            if (c != ']') {
+                if (c != '"') return PJ_BAIL;
+                for (;;) {                                        // p: a url's content
+                    const Str r = tstr(F, p);
+                    if (r.err) return r.err;
+                    n_urls++;
+                    url_bytes += r.dlen;
+                    // url k at word 5 + k (n_urls counts it already)
+                    if (n_urls <= TAPE_WORDS - 5) T[4 + n_urls] = tape_str(p, r);
+                    const uint64_t a = F.ld8(r.end);              // '"' then ']' or ',"'
+                    p = r.end + 2;
+                    c = (uint32_t)(a >> 8) & 0xFF;
+                    if (c == ']') break;
+                    if ((a & 0xFFFF00) != ((',' << 8) | ('"' << 16))) return PJ_BAIL;
+                    p++;
+                }
+            }
+            T_SEP();
+        }
+        if (more && last < 5 && k8 == KP_TAGS) {
+            last = 5;
+            flags |= PJ_PET_HAS_TAGS;
+            const uint32_t c = (uint32_t)k16 & 0xFF;              // the byte after '['
+            p += 9;                                               // past it
+            if (c != ']') {
+                if (c != '{') return PJ_BAIL;
+                for (;;) {                                        // p: a tag's body
+                    int64_t tid;
+                    uint32_t tfl, nq = 0;
+                    uint64_t a;
+                    Str nr{0, 0, 0, false};
+                    const int e = tsub(F, p, tid, tfl, nq, nr, a);
+                    if (e) return e;
+                    const uint32_t tl = (tfl & PJ_SUB_HAS_NAME) ? nr.dlen : 0;
+                    n_tags++;
+                    tag_bytes += tl;
+                    // tag k at words 5 + urls + 2k, + 1 (n_tags counts it already)
+                    if (n_urls + 2 * n_tags <= TAPE_WORDS - 5) {
+                        T[3 + n_urls + 2 * n_tags] = (uint64_t)tid;
+                        T[4 + n_urls + 2 * n_tags] = (tl ? tape_str(nq, nr) : 0) | ((uint64_t)(tfl & 3) << 49);
+                    }
+                    p += 2;                                       // '}' then ']' or ',{'
+                    if (((a >> 8) & 0xFF) == ']') break;
+                    if ((a & 0xFFFF00) != ((',' << 8) | ('{' << 16))) return PJ_BAIL;
+                    p++;
+                }
+            }
+            T_SEP();
+        }
+        if (more && last < 6 && k8 == KP_STATUS && (k16 & 0xFFFFull) == pack8(":\"", 2)) {
+            last = 6;
+            const uint32_t q = p + 10;
+            const uint64_t x = F.ld8(q), y = F.ld8(q + 8);
+            if (x == pack8("availabl", 8) && (y & 0xFFFF) == pack8("e\"", 2)) {
+                status = PJ_STATUS_AVAILABLE;
+                p = q + 10;
+            } else if (x == pack8("pending\"", 8)) {
+                status = PJ_STATUS_PENDING;
+                p = q + 8;
+            } else if ((x & 0xFFFFFFFFFFull) == pack8("sold\"", 5)) {
+                status = PJ_STATUS_SOLD;
+                p = q + 5;
+            } else {
+                const Str r = tstr(F, q);
+                if (r.err) return r.err;
+                return r.esc ? PJ_BAIL : PJ_REC_BAD_STATUS;        // (the enum's @JsonCreator rejects it)
+            }
+            T_SEP();
+        }
+        if (!more) break;
+        // an unknown property is skipped; a known key here is repeated, out
+        // of order or in another shape
+        if (known8(k8)) return PJ_BAIL;
+        const uint64_t r = fskip(F, p);
+        if ((uint32_t)r) return (int)(uint32_t)r;
+        p = (uint32_t)(r >> 32);
+        T_SEP();
+    }
+#undef T_SEP
+    if (p + 1 != n) return PJ_BAIL;                               // trailing bytes: general rules
+    if (!(flags & PJ_PET_HAS_NAME)) return PJ_REC_MISSING_NAME;   // required (petstore.json:873-876)
+    if (!(flags & PJ_PET_HAS_PHOTOURLS)) return PJ_REC_MISSING_PHOTOURLS;
+    R.name_len = name_len; R.cat_len = cat_len; R.n_urls = n_urls; R.url_bytes = url_bytes;
+    R.n_tags = n_tags; R.tag_bytes = tag_bytes;
+    if (n_urls + 2 * n_tags > TAPE_WORDS - 5) return PJ_TAPE_FULL;
+    T[0] = (uint64_t)id;
+    T[1] = (uint64_t)cat_id;
+    T[2] = (uint64_t)flags | ((uint64_t)status << 8) | ((uint64_t)cat_fl << 16) | ((uint64_t)n_urls << 24) |
+           ((uint64_t)n_tags << 32);
+    return 0;
+}
 
 // Writing a line from its tape: the stores and copies of fline<true>, in the
 // same order, without walking the line again.  The first TAPE_PRE words come
@@ -2650,7 +2905,7 @@ __device__ __forceinline__ void dec_block(DecParams &P, const uint64_t b) {
                     // strings are scanned and checked byte class by byte
                     // class as the walk meets them: no bitmaps needed
                     const FLine F{(const PJ_LDS uint8_t *)(tile + s0), nullptr, s0, n};
-                    if constexpr (TAPE) code = fline<false, FLine, true>(F, r, nullptr, nullptr, Tape{P.tape + l, P.lines});
+                    if constexpr (TAPE) code = fline_tape(F, r, Tape{P.tape + l, P.lines});
                     else code = fline<false>(F, r, nullptr, nullptr);
                     if (TAPE && code == PJ_TAPE_FULL) {
                         longl = true;

@@ -633,3 +633,38 @@ def test_decode_long_line_bitmaps_at_word_and_round_edges(codec, shift):
                 lines.append(b'{"id":7,"category":{"id":1,"name":"c"},"name":"' + body[31:] + b'","photoUrls":[]}')
     data = b"\n".join(lines) + b"\n"
     assert_same(gpu_decode(codec, data, shift=shift), orc.decode(data))
+
+
+@pytest.mark.parametrize("tail", [b"\n", b""])
+def test_decode_validating_walk_edges(codec, tail):
+    """The per-thread walk's tokens at their edges, against the oracle:
+    integers of every length and sign, at and past the int64 limits, in each
+    place one may stand; strings whose stop byte (quote, escape, surrogate
+    pair, multi-byte character, control) falls at every offset of a 16-byte
+    step; empty lists and bodies; unknown properties between and after the
+    known ones, repeated and out-of-order keys."""
+    nums = [s + d for s in ("", "-") for d in ["0", "00", "7", "07"] + ["123456789012345678901234"[:k] for k in range(2, 25)]]
+    nums += ["9223372036854775807", "9223372036854775808", "-9223372036854775808", "-9223372036854775809",
+             "9999999999999999999", "1.5", "1e3", "-", "", "null", "1 ", "12345678}", "1]"]
+    lines = []
+    for v in nums:
+        lines += ['{"id":%s,"name":"n","photoUrls":[]}' % v, '{"id":%s}' % v,
+                  '{"category":{"id":%s},"name":"n","photoUrls":[]}' % v,
+                  '{"category":{"id":%s,"name":"c"},"name":"n","photoUrls":["u"],"tags":[{"id":%s},{"id":%s,"name":"t"}]}' % (v, v, v)]
+    stops = ['', '\\"', '\\u00e9', '\\u0001', '\\ud83d\\ude00', '\\ud83d', '\\udc00', '\\x', '\\u12g4', 'é', '€', '\U0001f600', '\x02']
+    for k in range(0, 36):
+        for st in stops:
+            s = "a" * k + st + "b" * (k % 5)
+            lines += ['{"id":1,"name":"%s","photoUrls":["%s","%s"],"status":"sold"}' % (s, s, s[:k]),
+                      '{"category":{"name":"%s"},"name":"","photoUrls":[],"tags":[{"name":"%s"},{},{"id":3,"name":"%s"}]}' % (s, s, s)]
+    keys = ['"id":5', '"category":{}', '"name":"x"', '"photoUrls":["p"]', '"tags":[]', '"status":"pending"', '"zz":1',
+            '"q":"s"', '"idx":true', '"names":null', '"status":"available"', '"status":"soldx"', '"status":"so\\u006cd"',
+            '"tags":[{}]', '"name":null', '"photoUrls":[ ]', '"id": 5']
+    rnd = random.Random(11)
+    for i in range(3000):
+        pick = [keys[j] for j in range(6) if rnd.random() < 0.85]
+        for _ in range(rnd.randrange(0, 3)):
+            pick.insert(rnd.randrange(0, len(pick) + 1), rnd.choice(keys))
+        lines.append("{" + ",".join(pick) + "}" + ("" if i % 17 else "x"))
+    data = "\n".join(lines).encode("utf-8") + tail
+    assert_same(gpu_decode(codec, data), orc.decode(data))
