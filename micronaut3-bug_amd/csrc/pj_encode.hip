@@ -2063,53 +2063,103 @@ __global__ __launch_bounds__(BT) void k_enc_measure(EncParams P) {
     }
 }
 
+// A block's records written once each is measured: thread t holds record t
+// of `live`, n bytes long; pre is its offset in the block and agg the block's
+// length.  Runs of records that fit the LDS tile are built there (emit(sink),
+// LdsSinkU) and leave with aligned 16-byte stores (tile_copy_out), the first
+// run while the look-back resolves; a record larger than the tile is written
+// by its own thread (SectorSink).  Bytes past the capacity are not written;
+// the last block stores the total.  All threads call.
+template <int BT, int TILE> struct RunTile {
+    uint8_t bytes[TILE + 32];                    // tile_copy_out reads 32 bytes past
+    uint64_t base, end;
+};
+template <int BT, int TILE, class P, class F>
+__device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uint64_t b, uint64_t nblk, uint32_t live,
+                                          uint64_t pre, uint64_t n, uint64_t agg, F &&emit) {
+    const uint32_t t = threadIdx.x;
+    const uint64_t end = pre + n;
+    if (t == 0) lb_publish(p.state, b, agg);
+    bool placed = false;                     // sh.base holds the block's offset
+    uint64_t at = 0;                         // block offset of the run's first record
+    for (uint32_t r0 = 0; r0 < live;) {
+        // the run: records r0 .. r0 + k - 1 end within the tile
+        const bool mine = t >= r0 && t < live && end - at <= (uint64_t)TILE;
+        if (mine && !p.count_only) {
+            LdsSinkU ls{sh.bytes, (uint32_t)(pre - at), (uint32_t)(end - at)};
+            emit(ls);
+        }
+        if (!placed) {
+            placed = true;
+            if (t < 64) {
+                const uint64_t excl = lb_resolve(p.state, b, agg);
+                if (t == 0) {
+                    sh.base = excl;
+                    if (b == nblk - 1) *p.total = excl + agg;
+                }
+            }
+        }
+        const uint32_t k = (uint32_t)__syncthreads_count(mine);    // (the run's tile is built, the base known)
+        if (p.count_only) return;
+        const uint64_t base = sh.base;
+        if (k == 0) {                        // record r0 is larger than the tile
+            if (t == r0) {
+                if (base + end <= p.cap) {
+                    SectorSink xs;
+                    xs.init(p.out + base + pre);
+                    emit(xs);
+                    xs.finish();
+                }
+                sh.end = end;
+            }
+        } else if (t == r0 + k - 1) sh.end = end;
+        __syncthreads();
+        const uint64_t stop = sh.end;
+        if (k) {
+            const uint64_t hi = min(base + stop, p.cap);
+            if (base + at < hi) tile_copy_out<BT>(sh.bytes, p.out, base + at, base + at, hi, t);
+        }
+        at = stop;
+        r0 += k ? k : 1;
+        __syncthreads();                     // the tile and sh.end are free for the next run
+    }
+}
+
 // One thread per output record, blocks of BT records claimed by ticket:
 // pretty-printed output (PRETTY), and the records a selection names
 // (P.sel: output record j is column record sel[j]; compact or pretty).  Each
 // thread measures its record from global memory, a block scan places the
-// records, the look-back gives the block's offset, and each thread writes
-// its record with exact stores.  (Staging a block's output in LDS for
-// aligned stores measured slower: these blocks rarely fit a tile that
-// leaves room for other workgroups.)  Records that would end past the
-// capacity are not written; the last block stores the total.
-template <int BT, bool PRETTY>
-__global__ __launch_bounds__(BT) void k_encode_rows(EncParams P) {
+// records, and they leave in runs through the tile.  Bound by the latency of
+// each record's reads.  A third of 2M nested records by status: 0.51 -> 0.43 ms
+// against 32-byte sectors stored by each thread; 2M flat records pretty:
+// 0.27 -> 0.16 ms.
+template <int BT, bool PRETTY, int TILE>
+__global__ __launch_bounds__(BT, 4) void k_encode_rows(EncParams P) {
     stamp_start(P.stamp);
+    __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
     __shared__ uint64_t sh_scan[BT / 64 + 2];
-    __shared__ uint64_t sh_b, sh_base;
+    __shared__ uint64_t sh_b;
     const ColSrc XG{P.c.name_bytes, P.c.cat_name_bytes, P.c.url_bytes, P.c.tag_name_bytes, 0, 0, 0, 0};
     const uint32_t t = threadIdx.x;
     if (t == 0) sh_b = atomicAdd(P.ticket, 1ull);
     __syncthreads();
     const uint64_t b = sh_b, nblk = (P.n + BT - 1) / BT;
     const uint64_t j = b * BT + t;
-    const bool live = j < P.n;
+    const uint32_t live = (uint32_t)min((uint64_t)BT, P.n - b * BT);
     RecVals v{};
     RecItems ri{};
     CountSink cs;
-    if (live) {
+    auto emit = [&](auto &s) {
+        if constexpr (PRETTY) pp_rec(s, P, j, v);
+        else emit_rec<true, true>(s, P, XG, j, v, ri);
+    };
+    if (t < live) {
         v = load_rec<true>(P, P.sel ? P.sel[j] : j);
-        if (PRETTY) pp_rec(cs, P, j, v);
-        else emit_rec<true, true>(cs, P, XG, j, v, ri);
+        emit(cs);
     }
     uint64_t agg;
     const uint64_t pre = block_excl_scan<BT>(cs.n, sh_scan, &agg);
-    if (t < 64) {
-        const uint64_t excl = lookback(P.state, b, agg);
-        if (t == 0) {
-            sh_base = excl;
-            if (b == nblk - 1) *P.total = excl + agg;
-        }
-    }
-    __syncthreads();
-    if (P.count_only || !live) return;
-    const uint64_t at = sh_base + pre;
-    if (at + cs.n > P.cap) return;
-    SectorSink xs;
-    xs.init(P.out + at);
-    if (PRETTY) pp_rec(xs, P, j, v);
-    else emit_rec<true, true>(xs, P, XG, j, v, ri);
-    xs.finish();
+    emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
 }
 
 // The records whose status code is in the mask (bit s: status s, bit 3: no
@@ -2260,20 +2310,17 @@ __device__ __forceinline__ void m_rec(S &s, const ModelEncParams &P, uint64_t i,
 }
 
 // One thread per record in blocks of BT claimed by ticket: the values are
-// loaded once, measured and placed by a block scan; then runs of records
-// that fit the LDS tile are built there and leave with aligned 16-byte
-// stores (tile_copy_out), the first run while the look-back resolves.  A
-// record larger than the tile is written by its thread (SectorSink).
-// Bound by the instructions of the two passes over each record and by the
-// latency of its scattered string reads.  1M Orders (178 MB moved) 0.189 ->
-// 0.103 ms and 1M Users 0.344 -> 0.237 ms against a second pass that loaded
-// the values again and stored 32-byte sectors from each thread.
+// loaded once, measured, placed by a block scan and written in runs through
+// the tile.  Bound by the instructions of the two passes over each record and
+// by the latency of its scattered string reads.  1M Orders (178 MB moved)
+// 0.189 -> 0.103 ms and 1M Users 0.344 -> 0.237 ms against a second pass that
+// loaded the values again and stored 32-byte sectors from each thread.
 template <int MODEL, bool PRETTY, int BT, int TILE>
 __global__ __launch_bounds__(BT, 4) void k_encode_model(ModelEncParams P) {
     stamp_start(P.stamp);
-    __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 32];    // tile_copy_out reads 32 bytes past
+    __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
     __shared__ uint64_t sh_scan[BT / 64 + 2];
-    __shared__ uint64_t sh_b, sh_base, sh_end;
+    __shared__ uint64_t sh_b;
     const uint32_t t = threadIdx.x;
     if (t == 0) sh_b = atomicAdd(P.ticket, 1ull);
     __syncthreads();
@@ -2282,56 +2329,14 @@ __global__ __launch_bounds__(BT, 4) void k_encode_model(ModelEncParams P) {
     const uint32_t live = (uint32_t)min((uint64_t)BT, P.n - b * BT);
     MVals V;
     CountSink cs;
+    auto emit = [&](auto &s) { m_rec<MODEL, PRETTY>(s, P, i, V); };
     if (t < live) {
         V = m_load<MODEL>(P, i);
-        m_rec<MODEL, PRETTY>(cs, P, i, V);
+        emit(cs);
     }
     uint64_t agg;
-    const uint64_t pre = block_excl_scan<BT>(cs.n, sh_scan, &agg), end = pre + cs.n;
-    if (t == 0) lb_publish(P.state, b, agg);
-    bool placed = false;                     // sh_base holds the block's offset
-    uint64_t at = 0;                         // block offset of the run's first record
-    for (uint32_t r0 = 0; r0 < live;) {
-        // the run: records r0 .. r1 - 1 end within the tile
-        const bool mine = t >= r0 && t < live && end - at <= (uint64_t)TILE;
-        if (mine && !P.count_only) {
-            LdsSinkU ls{tile, (uint32_t)(pre - at), (uint32_t)(end - at)};
-            m_rec<MODEL, PRETTY>(ls, P, i, V);
-        }
-        if (!placed) {
-            placed = true;
-            if (t < 64) {
-                const uint64_t excl = lb_resolve(P.state, b, agg);
-                if (t == 0) {
-                    sh_base = excl;
-                    if (b == nblk - 1) *P.total = excl + agg;
-                }
-            }
-        }
-        const uint32_t k = (uint32_t)__syncthreads_count(mine);    // (the run's tile is built, the base known)
-        if (P.count_only) return;
-        const uint64_t base = sh_base;
-        if (k == 0) {                        // record r0 is larger than the tile
-            if (t == r0) {
-                if (base + end <= P.cap) {
-                    SectorSink xs;
-                    xs.init(P.out + base + pre);
-                    m_rec<MODEL, PRETTY>(xs, P, i, V);
-                    xs.finish();
-                }
-                sh_end = end;
-            }
-        } else if (t == r0 + k - 1) sh_end = end;
-        __syncthreads();
-        const uint64_t stop = sh_end;
-        if (k) {
-            const uint64_t hi = min(base + stop, P.cap);
-            if (base + at < hi) tile_copy_out<BT>(tile, P.out, base + at, base + at, hi, t);
-        }
-        at = stop;
-        r0 += k ? k : 1;
-        __syncthreads();                     // the tile and sh_end are free for the next run
-    }
+    const uint64_t pre = block_excl_scan<BT>(cs.n, sh_scan, &agg);
+    emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
 }
 
 __global__ void k_add_u64(uint64_t *p, uint64_t n, uint64_t v) {
@@ -2544,12 +2549,11 @@ hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t st) {
     return hipGetLastError();
 }
 
-// 512-record blocks: measured fastest (256 with three workgroups per CU
-// about the same; 128 and 64 slower, as more blocks chain their look-backs)
-#ifndef PJ_ENC_ROWS_BT
-#define PJ_ENC_ROWS_BT 512
-#endif
-constexpr int ENC_PRETTY_BT = PJ_ENC_ROWS_BT;
+// 256-record blocks with a 39 KiB tile, four workgroups per CU.  A third of 2M
+// nested records / 2M flat records pretty: 0.428 / 0.163 ms; 512 records and
+// 78 KiB 0.437 / 0.152, 128 and 19 KiB 0.431 / 0.232, 512 and 52 KiB (three
+// runs per block) 0.522 / 0.180.
+constexpr int ENC_PRETTY_BT = 256, ENC_ROWS_TILE = 39 * 1024;
 int pj_encode_pretty_records() { return ENC_PRETTY_BT; }
 
 constexpr int ENC_SEL_BT = 256, ENC_SEL_R = 16;
@@ -2557,10 +2561,10 @@ constexpr int ENC_SEL_BT = 256, ENC_SEL_R = 16;
 hipError_t pj_launch_encode_rows(const EncParams &P, bool pretty, hipStream_t st) {
     const uint64_t nblk = (P.n + ENC_PRETTY_BT - 1) / ENC_PRETTY_BT;
     if (pretty)
-        hipLaunchKernelGGL((pj::k_encode_rows<ENC_PRETTY_BT, true>), dim3((unsigned)nblk),
+        hipLaunchKernelGGL((pj::k_encode_rows<ENC_PRETTY_BT, true, ENC_ROWS_TILE>), dim3((unsigned)nblk),
                            dim3(ENC_PRETTY_BT), 0, st, P);
     else
-        hipLaunchKernelGGL((pj::k_encode_rows<ENC_PRETTY_BT, false>), dim3((unsigned)nblk),
+        hipLaunchKernelGGL((pj::k_encode_rows<ENC_PRETTY_BT, false, ENC_ROWS_TILE>), dim3((unsigned)nblk),
                            dim3(ENC_PRETTY_BT), 0, st, P);
     return hipGetLastError();
 }
