@@ -243,10 +243,14 @@ __host__ __device__ __forceinline__ uint64_t ld_tail(const uint8_t *p, int n) {
 }
 
 constexpr uint64_t ONES = 0x0101010101010101ull;
+// Flipping bit 1 takes '"' (0x22) to 0x20, keeps every control below 0x20 and
+// leaves nothing else below 0x21: one comparison finds the quotes and the
+// controls together.
+constexpr uint64_t QFLIP = 0x0202020202020202ull;
 // Nonzero iff some byte of x needs an output escape (< 0x20, '"', '\\').
 __device__ __forceinline__ uint64_t special64(uint64_t x) {
-    const uint64_t q = x ^ (0x22 * ONES), b = x ^ (0x5C * ONES);
-    return (((x - 0x20 * ONES) & ~x) | ((q - ONES) & ~q) | ((b - ONES) & ~b)) & (0x80 * ONES);
+    const uint64_t y = x ^ QFLIP, b = x ^ (0x5C * ONES);
+    return (((y - 0x21 * ONES) & ~y) | ((b - ONES) & ~b)) & (0x80 * ONES);
 }
 
 // ------------------------------------------------------- reading JSON
@@ -284,9 +288,8 @@ __device__ __forceinline__ int hex4(uint32_t x) {
 // (bits above it may be set too: borrows only run upwards from a byte that
 // is flagged itself).
 __device__ __forceinline__ uint64_t str_stop8(uint64_t x) {
-    constexpr uint64_t ONE = 0x0101010101010101ull;
-    const uint64_t q = x ^ (0x22 * ONE), b = x ^ (0x5C * ONE);
-    return (((q - ONE) & ~q) | ((b - ONE) & ~b) | (x - 0x20 * ONE) | x) & (0x80 * ONE);
+    const uint64_t b = x ^ (0x5C * ONES);
+    return (((b - ONES) & ~b) | ((x ^ QFLIP) - 0x21 * ONES) | x) & (0x80 * ONES);
 }
 // The same for '"' and '\\' only.
 __device__ __forceinline__ uint64_t quote_bs8(uint64_t x) {

@@ -205,11 +205,8 @@ __device__ __forceinline__ void emit_long(CountSink &s, int64_t v) {
 // or '\\'); exact per byte, unlike special64's "any" test.
 __device__ __forceinline__ uint64_t special_mask(uint64_t x) {
     constexpr uint64_t L7 = 0x7F7F7F7F7F7F7F7Full, H = 0x8080808080808080ull;
-    const uint64_t lo = x & L7;
-    const uint64_t lt20 = ~((lo + 0x6060606060606060ull) | x) & H;                 // < 0x20
-    const uint64_t q = (x ^ (0x22 * ONES)) & L7, bsl = (x ^ (0x5C * ONES)) & L7;
-    const uint64_t eq = ~(((q + L7) | (x ^ (0x22 * ONES))) & ((bsl + L7) | (x ^ (0x5C * ONES)))) & H;
-    return lt20 | eq;
+    const uint64_t y = x ^ QFLIP, b = x ^ (0x5C * ONES);                            // (y < 0x21: a control or '"')
+    return ~((((y & L7) + 0x5F * ONES) | y) & (((b & L7) + L7) | b)) & H;
 }
 // The escape of byte c (which needs one) as up to 6 bytes, formed without
 // branches: \" \\ \b \t \n \f \r, else \u00XX (hex digits a-f in the case
