@@ -96,6 +96,9 @@ struct pj_ctx {
     // nested encodes since one listed large records: while below BIG_RECENT,
     // k_enc_big follows the pass without waiting for its count
     int big_since = 1 << 20;
+    // Pet decodes since one with lines over the tile: while below BIG_RECENT,
+    // the large-tile kernels run with the others, not in a second attempt
+    int over_since = 1 << 20;
     uint64_t scan_zero = 0;       // leading words of `scan` known to be zero (left so by the last encode)
     uint64_t *stamps = nullptr;   // MAX_EV clock stamps of the call's launches (pinned, after the 64 result words)
     double ticks_per_ms = 1e5;    // of the device's wall clock
@@ -1322,11 +1325,14 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     P.dq_count = reinterpret_cast<unsigned long long *>(X + 13);
     P.long_count = reinterpret_cast<unsigned long long *>(X + 14);
     P.bticket = reinterpret_cast<unsigned long long *>(X + 15);
+    P.over_count = reinterpret_cast<unsigned long long *>(X + 23);
+    P.big_tile = ctx->over_since < BIG_RECENT;
     P.long_list = P.dq + lines + 8;
     P.lpos = reinterpret_cast<uint32_t *>(P.long_list + lines);
     P.bm_count = reinterpret_cast<unsigned long long *>(P.long_list + lines + w_lpos);
     P.bm_list = P.long_list + lines + w_lpos + 2;
     P.order_by_id = 1;
+    const int n_ev0 = ctx->n_ev;
     for (;;) {
         FillRanges R{};
         if (split) {
@@ -1335,12 +1341,13 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
         } else R.add(P.state_parse, gp * VLB_WORDS, 0);
         R.add(X + 1, 1, 0);      // the parse ticket / give-up word
         R.add(X + 3, 13, 0);     // totals and counters
+        R.add(X + 23, 1, 0);     // lines over the tile
         if (!lines) {            // the offset arrays still start with 0
             uint64_t *heads[6] = {out->name_off, out->cat_name_off, out->photo_off, out->tag_off, out->url_off,
                                   out->tag_name_off};
             R.k = 0;
             for (uint64_t *h : heads) R.add(h, 1, 0);
-            R.add(X + 3, 13, 0);
+            R.add(X + 3, 21, 0);
         }
         PJ_HIP(pj_launch_fill_ranges(R, ctx->stream, mark(ctx)));
         if (lines) {
@@ -1357,13 +1364,20 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
             P.stamp = mark(ctx);
             PJ_HIP(pj_launch_dec_errcode(P, ctx->stream));
         }
-        PJ_HIP(pj_launch_publish(ctx->pinned, X, 13, 0, -1, ctx->stream, mark(ctx)));
+        PJ_HIP(pj_launch_publish(ctx->pinned, X, 24, 0, -1, ctx->stream, mark(ctx)));
         PJ_HIP(hipStreamSynchronize(ctx->stream));
+        if (split && lines && ctx->pinned[23] && !P.big_tile) {
+            // lines over the tile were left unread: once more, with the large tile
+            P.big_tile = 1;
+            ctx->n_ev = n_ev0;
+            continue;
+        }
         if (!P.order_by_id || ctx->pinned[1] == 0) break;
         P.order_by_id = 0;
         ctx->n_ev = 0;
     }
     finish_timing(ctx);
+    if (split) ctx->over_since = ctx->pinned[23] ? 0 : std::min(ctx->over_since + 1, 1 << 20);
     const uint64_t *T = ctx->pinned + 4;
     res->n_general = lines ? ctx->pinned[12] : 0;
     res->n_lines = lines;

@@ -3127,7 +3127,12 @@ __global__ __launch_bounds__(BT, BM ? 2 : 3) void k_dec_block(DecParams P) {
 // one the walk does not recognise, by the general parser on one thread).
 // Its 8 counters go to tape words 0-7, its code and kind to its info word;
 // LK_DEFER stays set for k_dec_fixup.
-template <int TILE>
+// Lines over the tile are counted (P.over_count) and left to the instance
+// with the large tile (MIN: the small one), one line per CU at a time, which
+// the host launches once a call has counted some: read by one thread from
+// global memory, a line of 38 KB took 30 ms.  Past the large tile that
+// thread reads them.
+template <int TILE, int MIN>
 __global__ __launch_bounds__(64) void k_dec_measure_long(DecParams P) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
     __shared__ uint64_t spec[TILE / 64 + 1];
@@ -3143,6 +3148,17 @@ __global__ __launch_bounds__(64) void k_dec_measure_long(DecParams P) {
         const uint64_t a0 = gs & ~15ull, tb = min(ge, P.len) - a0;
         const uint32_t s0 = (uint32_t)(gs - a0);
         LineRec r{0, 0, 0, 0, 0, 0, 0, 0};
+        if (MIN ? tb <= (uint64_t)MIN : tb > (uint64_t)TILE) {
+            if (!MIN) {
+                // it counts as nothing until the large-tile instance reads it
+                if (t < PJ_DEC_NCNT) P.tape[t * L + l] = 0;
+                if (t == 0) {
+                    P.lpos[PJ_DEC_NCNT * L + l] = LK_DEFER | LK_WAVE;
+                    atomicAdd(P.over_count, 1ull);
+                }
+            }
+            continue;
+        }
         int code = 0;
         bool general = false, bad = false;
         LineInfo Li;
@@ -3359,7 +3375,9 @@ __global__ __launch_bounds__(BT, 2) void k_dec_write(DecParams P) {
 // the tape holds), one 64-thread workgroup per line at a time: the line is
 // tiled into LDS with its bitmaps and written by the wave-parallel walk.
 // Lines of the general parser are read again from the input by one thread.
-template <int TILE, int LPB>
+// The instance with the large tile (MIN: the small one) writes the lines over
+// the small tile.
+template <int TILE, int LPB, int MIN>
 __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
     stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
@@ -3375,6 +3393,9 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
         const uint32_t n = (uint32_t)(ge - 1 - gs);
         const uint32_t info = __builtin_amdgcn_readfirstlane(P.lpos[PJ_DEC_NCNT * L + l]);
         if (info & 0xFF) continue;                  // a deferred line found invalid
+        if (MIN ? ((info & LK_GENERAL) || min(ge, P.len) - (gs & ~15ull) <= (uint64_t)MIN)
+                : !(info & LK_GENERAL) && min(ge, P.len) - (gs & ~15ull) > (uint64_t)TILE)
+            continue;                               // the other instance's
         if (info & LK_GENERAL) {
             // the general parser, from the input (the measuring walk, then the writing walk)
             if (threadIdx.x == 0) {
@@ -3526,6 +3547,8 @@ constexpr int DEC_IDX_BT = 256, DEC_IDX_R = PJ_DEC_IDX_R, DEC_LINE_BT = PJ_DEC_L
 constexpr int DEC_WTILE = PJ_DEC_WTILE_KB * 1024;
 // The bitmap-free validating pass: 30 KiB keeps it under 32 KiB of LDS.
 constexpr int DEC_FTILE = PJ_DEC_WTILE_KB * 1024;
+// The large tile for single lines over DEC_TILE: with its bitmaps 150 KiB of LDS.
+constexpr int DEC_BIGTILE = 120 * 1024;
 static_assert(DEC_WTILE >= 4 * PJ_DEC_LONG, "fast lines (at most DEC_LONG bytes) fit the writer's tile");
 
 int pj_dec_index_block() { return DEC_IDX_BT * DEC_IDX_R; }
@@ -3603,8 +3626,13 @@ hipError_t pj_launch_dec_write(const DecParams &P, hipStream_t st) {
 }
 
 hipError_t pj_launch_dec_long(const DecParams &P, hipStream_t st) {
-    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, DEC_LPB>), dim3((unsigned)std::min<uint64_t>(1024, P.lines)), dim3(64), 0,
-                       st, P);
+    const unsigned g = (unsigned)std::min<uint64_t>(1024, P.lines);
+    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, DEC_LPB, 0>), dim3(g), dim3(64), 0, st, P);
+    if (P.big_tile) {
+        DecParams Q = P;
+        Q.stamp = nullptr;
+        hipLaunchKernelGGL((pj::k_dec_long<DEC_BIGTILE, DEC_LPB, DEC_TILE>), dim3(g), dim3(64), 0, st, Q);
+    }
     return hipGetLastError();
 }
 
@@ -3615,8 +3643,10 @@ hipError_t pj_launch_dec_parse(const DecParams &P, hipStream_t st) {
         // lines it deferred, then its offsets corrected for them
         hipLaunchKernelGGL((pj::k_dec_block<DEC_LINE_BT, DEC_FTILE, DEC_LONG, DEC_LPB, true, false>), dim3((unsigned)g),
                            dim3(DEC_LINE_BT), 0, st, P);
-        hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_TILE>), dim3((unsigned)std::min<uint64_t>(1024, P.lines)), dim3(64), 0,
-                           st, P);
+        const unsigned gl = (unsigned)std::min<uint64_t>(1024, P.lines);
+        hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_TILE, 0>), dim3(gl), dim3(64), 0, st, P);
+        if (P.big_tile)
+            hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_BIGTILE, DEC_TILE>), dim3(gl), dim3(64), 0, st, P);
         hipLaunchKernelGGL((pj::k_dec_fixup<DEC_LINE_BT, DEC_LPB>), dim3((unsigned)(g < 1024 ? g : 1024)),
                            dim3(DEC_LINE_BT), 0, st, P);
     } else

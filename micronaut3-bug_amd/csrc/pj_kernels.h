@@ -131,6 +131,8 @@ struct DecParams {
     uint64_t nblocks;          // line blocks of the validating kernel
     uint64_t *long_list;       // lines read by a whole wave, written by k_dec_long
     unsigned long long *long_count;
+    unsigned long long *over_count;   // deferred lines longer than the tile
+    int big_tile;              // 1: those lines are read by the large-tile instances (else left unread)
     unsigned long long *bticket;  // block ticket of the scan kernel
     // array documents: the frame's scalars (0 first non-whitespace byte,
     // 1 last non-whitespace byte + 1, 2 the close, 3 separators, 4 frame

@@ -668,3 +668,44 @@ def test_decode_validating_walk_edges(codec, tail):
         lines.append("{" + ",".join(pick) + "}" + ("" if i % 17 else "x"))
     data = "\n".join(lines).encode("utf-8") + tail
     assert_same(gpu_decode(codec, data), orc.decode(data))
+
+
+@pytest.mark.parametrize("array", [False, True])
+def test_decode_lines_around_the_tiles(codec, array):
+    """A line of up to 31,744 bytes is read by a wave from the small tile, up
+    to 122,880 from the large one (in a second attempt, or at once for a while
+    after a call that met such a line), a longer one by one thread: lines on
+    both sides of each size, valid and invalid, of the wave's shape and of the
+    general parser's, alone and among ordinary lines; then calls without any."""
+    rnd = random.Random(4)
+    short = orc.encode(pj.generate(3, 300), pj.FORMAT_NDJSON).split(b"\n")[:-1]
+
+    def line(n, kind):
+        name = "".join(rnd.choice(["abcdefgh", '\\"', "\\u00e9", "é", "\\n", "\U0001f600"]) for _ in range(n // 8)).encode()
+        pre, post = b'{"id":%d,"name":"' % n, b'","photoUrls":["u"],"tags":[{"id":1,"name":"t"}],"status":"sold"}'
+        while len(pre) + len(name) + len(post) > n:          # whole tokens only
+            name = name[: len(name) - 400]
+            name = name[: name.rfind(b"abcdefgh")]
+        x = pre + name + b"z" * (n - len(pre) - len(name) - len(post)) + post
+        if kind == 1:
+            x = x.replace(b'"sold"', b'"lost"')
+        elif kind == 2:
+            x = x[: n // 2] + b"\x01" + x[n // 2 + 1:]
+        elif kind == 3:
+            x = b'{"x":[{}],' + x[1:]                         # general parser
+        return x
+    sizes = (31_700, 31_727, 31_728, 31_743, 31_744, 31_745, 40_000, 100_000, 122_863, 122_864, 122_880, 122_881, 150_000)
+    docs = [[line(n, k)] for n in (31_743, 31_745, 60_000) for k in range(4)]
+    docs += [short[:150] + [line(n, (i + j) % 4) for i, n in enumerate(sizes)] + short[150:] for j in (0, 1)]
+    docs += [short] * 3 + [short + [line(90_000, 0)]] + [short] * 20 + [[line(33_000, 0)] + short]
+    for lines in docs:
+        if array:
+            data = b"[" + b",".join(lines) + b"]"
+            t = torch.frombuffer(bytearray(data), dtype=torch.uint8).cuda()
+            cols, el, ec, res = codec.decode_array(t)
+            rc, *ref = orc.decode_array(data)
+            assert rc == pj.PJ_OK
+            assert_same((cols.to_host(), el.cpu().numpy().astype(np.uint64), ec.cpu().numpy(), res), ref)
+        else:
+            data = b"\n".join(lines) + b"\n"
+            assert_same(gpu_decode(codec, data), orc.decode(data))
