@@ -1214,8 +1214,7 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
             R.add(X, 16, 0);
             R.add(X + o_sidx, gidx, 0);
             if (array) {
-                R.add(X + o_arr, 1, ~0ull);      // first non-whitespace
-                R.add(X + o_arr + 1, 1, 0);
+                R.add(X + o_arr, 2, 0);
                 R.add(X + o_arr + 2, 1, ~0ull);  // the close
                 R.add(X + o_arr + 3, 5, 0);
             }

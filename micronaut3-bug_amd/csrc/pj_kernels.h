@@ -134,8 +134,7 @@ struct DecParams {
     unsigned long long *over_count;   // deferred lines longer than the tile
     int big_tile;              // 1: those lines are read by the large-tile instances (else left unread)
     unsigned long long *bticket;  // block ticket of the scan kernel
-    // array documents: the frame's scalars (0 first non-whitespace byte,
-    // 1 last non-whitespace byte + 1, 2 the close, 3 separators, 4 frame
+    // array documents: the frame's scalars (2 the close, 3 separators, 4 frame
     // ok, 5 block ticket), per-block summaries and entry states; array_doc
     // makes the line stages read each element's separator as its newline
     int array_doc;

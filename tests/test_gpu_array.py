@@ -190,3 +190,18 @@ def test_array_frame_words_per_thread(codec, size):
     assert len(doc) == size
     ref = orc.decode_array(doc)
     assert_same(doc, gpu_array(codec, doc), ref)
+
+
+@pytest.mark.parametrize("lead,trail", [(0, 0), (5, 3), (16383, 16385), (40_000, 1), (1, 1_200_000), (17_000_000, 100),
+                                        (7, 17_300_000)])
+def test_array_whitespace_around_the_frame(codec, lead, trail):
+    """The document's first and last bytes that are not whitespace come from
+    one word per block of the frame: whitespace over whole blocks (16 KiB, and
+    128 KiB past 16 MiB) and more than 64 of them before and after the array,
+    and a stray byte at either end, which breaks the frame."""
+    body = b'[{"name":"a","photoUrls":[]},{"name":"b","photoUrls":["u"]}]'
+    ws = np.frombuffer(b" \t\r\n", np.uint8)
+    rng = np.random.default_rng(lead + trail)
+    pre, post = ws[rng.integers(0, 4, lead)].tobytes(), ws[rng.integers(0, 4, trail)].tobytes()
+    for doc in (pre + body + post, b"x" + pre + body + post, pre + body + post + b"]", pre + post):
+        assert_same(doc, gpu_array(codec, doc), orc.decode_array(doc))
