@@ -1486,28 +1486,26 @@ struct FLineT {
             return;
         }
         if (!special) {
-            // runs between escapes go out whole; the next backslash (or the
-            // closing quote) is found 8 bytes at a time
-            uint8_t *dd = dst;
-            uint32_t x = q;
-            for (;;) {
-                uint32_t stop = x;
-                for (;;) {
-                    const uint64_t m = quote_bs8(ld8(stop));
-                    if (m) { stop += (uint32_t)__builtin_ctzll(m) >> 3; break; }
-                    stop += 8;
+            // the decoded bytes gather in a register and leave eight at a
+            // time: escapes are close together where there are many, and
+            // storing each run and each escape by itself took several
+            // scattered stores for a few bytes (k_dec_write of 250,000
+            // skewed lines 384 -> 347 us, of 3M lines 664 -> 652)
+            StoreSink o;
+            o.init(dst);
+            for (uint32_t x = q; x < r.end;) {
+                const uint64_t w = ld8(x), bs = w ^ (0x5C * ONES), m = (bs - ONES) & ~bs & (0x80 * ONES);
+                const uint32_t lim = min(8u, r.end - x);
+                const uint32_t run = m ? min((uint32_t)__builtin_ctzll(m) >> 3, lim) : lim;
+                if (run) o.put8(w, run);
+                x += run;
+                if (run < lim) {
+                    const Esc e = esc(x);
+                    o.put(e.out, e.k);
+                    x += e.adv;
                 }
-                stop = min(stop, r.end);
-                if (stop > x) {
-                    copy_from_lds(dd, s + x, stop - x);
-                    dd += stop - x;
-                }
-                if (stop >= r.end) break;
-                const Esc e = esc(stop);
-                st_tail(dd, e.out, (uint32_t)e.k);
-                dd += e.k;
-                x = stop + e.adv;
             }
+            o.finish();
             return;
         }
         // runs between escapes go out whole; the specials bitmap finds the
@@ -2124,7 +2122,9 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
 // token accepts, so reads need no bounds but the tile's own padding.
 // 3M lines (823 MB): k_dec_block 928 -> 734 us; 250,000 skewed
 // lines (137 MB, escape-heavy names): 740 -> 480 us.  (The next 16 bytes of a
-// string loaded while these are tested: no change, 772 against 770.)
+// string loaded while these are tested: no change, 772 against 770.  All stops
+// of 16 bytes taken from the bytes at hand, without reading again: 705 -> 768 us
+// with the long lines' measuring on the skewed lines.)
 
 // m (1..8) digits packed in x, first digit lowest
 __device__ __forceinline__ uint32_t digits8_dot(uint64_t x, uint32_t m) {

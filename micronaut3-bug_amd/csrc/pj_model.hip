@@ -942,23 +942,27 @@ __global__ __launch_bounds__(MD_TOPS) void k_mdec_scan_tops(ModelDecParams P) {
 }
 
 // The decoded string whose content starts at q of a staged record, len bytes
-// with its escapes decoded, to dst: runs between escapes go out whole.  The
-// counting pass has read it, so every escape is well formed.
-__device__ __forceinline__ void m_copy_esc(const MLds &L, uint32_t q, uint64_t len, uint8_t *dst) {
-    uint8_t *const end = dst + len;
-    while (dst < end) {
-        uint32_t stop = q;
-        uint64_t m;
-        while (!(m = quote_bs8(L.ld8(stop)))) stop += 8;
-        stop += (uint32_t)__builtin_ctzll(m) >> 3;
-        copy_from_lds(dst, L.s + q, stop - q);
-        dst += stop - q;
-        if (dst >= end) break;
-        const MEsc e = m_escape(L, stop, L.ld8(stop));
-        st_tail(dst, e.out, (uint32_t)e.k);
-        dst += e.k;
-        q = stop + e.adv;
+// with its escapes decoded, to dst: the bytes gather in a register and leave
+// eight at a time.  The counting pass has read it, so every escape is well
+// formed.
+__device__ __forceinline__ void m_copy_esc(const MLds &L, uint32_t q, uint32_t len, uint8_t *dst) {
+    StoreSink o;
+    o.init(dst);
+    for (uint32_t done = 0; done < len;) {
+        const uint64_t w = L.ld8(q), bs = w ^ (0x5C * ONES), m = (bs - ONES) & ~bs & (0x80 * ONES);
+        const uint32_t lim = min(8u, len - done);
+        const uint32_t run = m ? min((uint32_t)__builtin_ctzll(m) >> 3, lim) : lim;
+        if (run) o.put8(w, run);
+        q += run;
+        done += run;
+        if (run < lim) {
+            const MEsc e = m_escape(L, q, L.ld8(q));
+            o.put(e.out, e.k);
+            done += (uint32_t)e.k;
+            q += e.adv;
+        }
     }
+    o.finish();
 }
 
 // Bound by the scattered string stores (16-byte stores at any address).  1M
@@ -1043,7 +1047,7 @@ __global__ __launch_bounds__(BT) void k_mdec_write(ModelDecParams P) {
                     const MLds L{(const PJ_LDS uint8_t *)S.tile + (a - S.g0), 0};
                     const uint32_t q = (uint32_t)R.spos[k] + 1;
                     if (!((R.sesc >> k) & 1)) copy_from_lds(o.bytes[k] + s0, L.s + q, (uint32_t)R.slen[k]);
-                    else m_copy_esc(L, q, R.slen[k], o.bytes[k] + s0);
+                    else m_copy_esc(L, q, (uint32_t)R.slen[k], o.bytes[k] + s0);
                 }
             } else if (R.slen[k] && s1 <= o.cap_bytes[k]) {
                 MStore w(o.bytes[k] + s0);
