@@ -1292,7 +1292,6 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     P.err_code = err_code;
     P.err_cap = err_cap;
     P.lines = lines;
-    const uint64_t gp = (lines + pj_dec_parse_block() - 1) / pj_dec_parse_block();
     // the line tape (256 bytes per line), when it fits a modest bound;
     // with it the decode is split at the scan (the validating kernel
     // stores per-line offsets, the writers follow a block scan), without
@@ -1303,6 +1302,8 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
         P.tape = static_cast<uint64_t *>(ctx->tape.p);
     (void)hipGetLastError();
     const bool split = P.tape != nullptr;
+    P.lpb = split ? pj_dec_split_block(len, lines) : pj_dec_parse_block();
+    const uint64_t gp = (lines + P.lpb - 1) / P.lpb;
     // scan buffer: vector look-back words (single pass) or block totals,
     // bases and scan look-back words (split), then the deferred
     // error-code queue, then (split) the wave-line list, the per-line

@@ -3138,7 +3138,7 @@ __device__ __forceinline__ void dec_block(DecParams &P, const uint64_t b) {
 }
 
 template <int BT, int TILE, int LONG, int LPB = BT, bool TAPE = false, bool BM = true>
-__global__ __launch_bounds__(BT, BM ? 2 : 3) void k_dec_block(DecParams P) {
+__global__ __launch_bounds__(BT, BM || BT == 64 ? 2 : 3) void k_dec_block(DecParams P) {
     stamp_start(P.stamp);
     __shared__ uint64_t sh_blk;
     if (threadIdx.x == 0) sh_blk = P.order_by_id ? (uint64_t)blockIdx.x : atomicAdd(&P.tickets[1], 1ull);
@@ -3402,7 +3402,7 @@ __global__ __launch_bounds__(BT, 2) void k_dec_write(DecParams P) {
 // Lines of the general parser are read again from the input by one thread.
 // The instance with the large tile (MIN: the small one) writes the lines over
 // the small tile.
-template <int TILE, int LPB, int MIN>
+template <int TILE, int MIN>
 __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
     stamp_start(P.stamp);
     __shared__ __attribute__((aligned(16))) uint8_t tile[TILE + 64];
@@ -3426,7 +3426,7 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
             if (threadIdx.x == 0) {
                 uint64_t gp[PJ_DEC_NCNT];
 #pragma unroll
-                for (int k = 0; k < PJ_DEC_NCNT; k++) gp[k] = P.bbase[(l / LPB) * PJ_DEC_NCNT + k] + P.lpos[k * L + l];
+                for (int k = 0; k < PJ_DEC_NCNT; k++) gp[k] = P.bbase[(l / (uint32_t)P.lpb) * PJ_DEC_NCNT + k] + P.lpos[k * L + l];
                 const Src S{P.in, P.len, nullptr};
                 LineInfo Li;
                 run_line(P, S, gs, n, true, false, Li, nullptr);
@@ -3442,7 +3442,7 @@ __global__ __launch_bounds__(64) void k_dec_long(DecParams P) {
         __syncthreads();
         tile_bitmaps_wave<false>(tile, nw, spec, badm, 0, 0);  // the line is valid: specials only
         __syncthreads();
-        const uint64_t pb = l / LPB;
+        const uint64_t pb = l / (uint32_t)P.lpb;
         uint64_t base[PJ_DEC_NCNT];
         uint32_t rel[PJ_DEC_NCNT];
 #pragma unroll
@@ -3582,6 +3582,21 @@ int pj_dec_index_block() { return DEC_IDX_BT * DEC_IDX_R; }
 #endif
 constexpr int DEC_LPB = PJ_DEC_LPB;
 int pj_dec_parse_block() { return DEC_LPB; }
+// Blocks for lines that are long on average: one wave of 64 lines and a tile
+// of 18 KiB, eight workgroups per CU.  Blocks of 104 such lines are cut into
+// sub-tiles, whose other lines' lanes wait, and one escape-heavy line holds
+// both of their waves; blocks of 64 hold fewer.  Lines of 274 bytes on average
+// fit the large blocks whole.  The line lies where the large tile holds 104
+// average lines no longer: 200,000 lines of 273 / 293 / 313 / 403 / 533 bytes,
+// k_dec_block 92 / 125 / 153 / 166 / 173 us in large blocks, 92 / 126 / 139 /
+// 147 / 156 in small ones (k_dec_write 60 / 72 / 88 / 95 / 96 and 61 / 72 / 81 /
+// 84 / 87); 250,000 skewed lines 706 -> 608 and 346 -> 271 us; 3M lines of 274
+// bytes 720 and 637 in large, 757 and 670 in small ones.
+constexpr int DEC_SBT = 64, DEC_SLPB = 64, DEC_STILE = 18 * 1024;
+static_assert(DEC_STILE >= 4 * PJ_DEC_LONG, "fast lines fit the tile");
+int pj_dec_split_block(uint64_t len, uint64_t lines) {
+    return len > lines * (uint64_t)(DEC_FTILE / DEC_LPB) ? DEC_SLPB : DEC_LPB;
+}
 
 namespace pj {
 // Sets *flag when some line block spans PJ_DEC_MAX_BLOCK_SPAN bytes or more.
@@ -3645,35 +3660,45 @@ hipError_t pj_launch_dec_bscan(const DecParams &P, hipStream_t st) {
 }
 
 hipError_t pj_launch_dec_write(const DecParams &P, hipStream_t st) {
-    hipLaunchKernelGGL((pj::k_dec_write<DEC_LINE_BT, DEC_WTILE, DEC_LPB, DEC_LONG>), dim3((unsigned)P.nblocks), dim3(DEC_LINE_BT), 0,
-                       st, P);
+    if (P.lpb == DEC_SLPB)
+        hipLaunchKernelGGL((pj::k_dec_write<DEC_SBT, DEC_STILE, DEC_SLPB, DEC_LONG>), dim3((unsigned)P.nblocks), dim3(DEC_SBT),
+                           0, st, P);
+    else
+        hipLaunchKernelGGL((pj::k_dec_write<DEC_LINE_BT, DEC_WTILE, DEC_LPB, DEC_LONG>), dim3((unsigned)P.nblocks),
+                           dim3(DEC_LINE_BT), 0, st, P);
     return hipGetLastError();
 }
 
 hipError_t pj_launch_dec_long(const DecParams &P, hipStream_t st) {
     const unsigned g = (unsigned)std::min<uint64_t>(1024, P.lines);
-    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, DEC_LPB, 0>), dim3(g), dim3(64), 0, st, P);
+    hipLaunchKernelGGL((pj::k_dec_long<DEC_TILE, 0>), dim3(g), dim3(64), 0, st, P);
     if (P.big_tile) {
         DecParams Q = P;
         Q.stamp = nullptr;
-        hipLaunchKernelGGL((pj::k_dec_long<DEC_BIGTILE, DEC_LPB, DEC_TILE>), dim3(g), dim3(64), 0, st, Q);
+        hipLaunchKernelGGL((pj::k_dec_long<DEC_BIGTILE, DEC_TILE>), dim3(g), dim3(64), 0, st, Q);
     }
     return hipGetLastError();
 }
 
 hipError_t pj_launch_dec_parse(const DecParams &P, hipStream_t st) {
-    const uint64_t g = (P.lines + DEC_LPB - 1) / DEC_LPB;
+    const uint64_t g = P.nblocks;
     if (P.tape) {
         // every block without bitmaps (five workgroups per CU), then the
         // lines it deferred, then its offsets corrected for them
-        hipLaunchKernelGGL((pj::k_dec_block<DEC_LINE_BT, DEC_FTILE, DEC_LONG, DEC_LPB, true, false>), dim3((unsigned)g),
-                           dim3(DEC_LINE_BT), 0, st, P);
+        const bool sm = P.lpb == DEC_SLPB;
+        if (sm)
+            hipLaunchKernelGGL((pj::k_dec_block<DEC_SBT, DEC_STILE, DEC_LONG, DEC_SLPB, true, false>), dim3((unsigned)g),
+                               dim3(DEC_SBT), 0, st, P);
+        else
+            hipLaunchKernelGGL((pj::k_dec_block<DEC_LINE_BT, DEC_FTILE, DEC_LONG, DEC_LPB, true, false>), dim3((unsigned)g),
+                               dim3(DEC_LINE_BT), 0, st, P);
         const unsigned gl = (unsigned)std::min<uint64_t>(1024, P.lines);
         hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_TILE, 0>), dim3(gl), dim3(64), 0, st, P);
         if (P.big_tile)
             hipLaunchKernelGGL((pj::k_dec_measure_long<DEC_BIGTILE, DEC_TILE>), dim3(gl), dim3(64), 0, st, P);
-        hipLaunchKernelGGL((pj::k_dec_fixup<DEC_LINE_BT, DEC_LPB>), dim3((unsigned)(g < 1024 ? g : 1024)),
-                           dim3(DEC_LINE_BT), 0, st, P);
+        const dim3 gf((unsigned)(g < 1024 ? g : 1024));
+        if (sm) hipLaunchKernelGGL((pj::k_dec_fixup<DEC_SBT, DEC_SLPB>), gf, dim3(DEC_SBT), 0, st, P);
+        else hipLaunchKernelGGL((pj::k_dec_fixup<DEC_LINE_BT, DEC_LPB>), gf, dim3(DEC_LINE_BT), 0, st, P);
     } else
         hipLaunchKernelGGL((pj::k_dec_block<DEC_LINE_BT, DEC_TILE, DEC_LONG, DEC_LPB, false>), dim3((unsigned)g),
                            dim3(DEC_LINE_BT), 0, st, P);

@@ -129,6 +129,7 @@ struct DecParams {
     uint64_t *bm_list;         // split decode: blocks holding deferred lines (nblocks entries)
     unsigned long long *bm_count;  // [0] blocks in bm_list, [1] unused
     uint64_t nblocks;          // line blocks of the validating kernel
+    int lpb;                   // lines per block: pj_dec_split_block's with the tape, else pj_dec_parse_block's
     uint64_t *long_list;       // lines read by a whole wave, written by k_dec_long
     unsigned long long *long_count;
     unsigned long long *over_count;   // deferred lines longer than the tile
@@ -228,6 +229,8 @@ int pj_dec_index_block();
 // u64); resolved once per device, with that device current.
 hipError_t pj_noalloc_scratch_init(int device, uint64_t **ptr);
 int pj_dec_parse_block();
+// Lines per block of the split decode of `lines` lines in len bytes.
+int pj_dec_split_block(uint64_t len, uint64_t lines);
 // The Pet decode keeps each line's output offsets inside its line block as
 // 32-bit values, so the bytes of a block's lines must stay below 4 GiB (a
 // line of 4 GiB or more is refused with them).  Block b holds lines

@@ -709,3 +709,29 @@ def test_decode_lines_around_the_tiles(codec, array):
         else:
             data = b"\n".join(lines) + b"\n"
             assert_same(gpu_decode(codec, data), orc.decode(data))
+
+
+@pytest.mark.parametrize("extra", [0, 40])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 103, 104, 105, 128, 129, 1000])
+def test_decode_block_sizes_by_average_line(codec, n, extra):
+    """Lines of up to 295 bytes on average are decoded in blocks of 104, longer
+    ones in blocks of 64 with a smaller tile: counts around both blocks' edges,
+    ordinary lines with deferred (long, full-tape), general, invalid and blank
+    ones first, last and next to each other in a block of either size."""
+    rnd = random.Random(n + extra)
+    base = orc.encode(pj.generate(3, n, seed=n), pj.FORMAT_NDJSON).split(b"\n")[:-1]
+    pad = b'{"zz":"' + b"q" * extra + b'",' if extra else b"{"
+    lines = [pad + x[1:] for x in base]
+    odd = [b'{"name":"' + b'ab\\n\xc3\xa9' * 250 + b'","photoUrls":["u"]}',
+           b'{"name":"t","photoUrls":[' + b",".join([b'"u"'] * 40) + b"]}", b'{ "name":"g","photoUrls":[]}', b"", b'{"name":1}',
+           b'{"name":"x\x01","photoUrls":[]}']
+    plain = len(b"\n".join(lines)) > 295 * n
+    for places in ([], [0, n - 1], [62, 63, 64, 103, 104], list(range(60, 68)) + [rnd.randrange(n) for _ in range(5)]):
+        doc = list(lines)
+        for p in places:
+            if p < n:
+                doc[p] = rnd.choice(odd)
+        data = b"\n".join(doc) + b"\n"
+        if not places and n > 1:
+            assert plain == (extra > 0)
+        assert_same(gpu_decode(codec, data), orc.decode(data))
