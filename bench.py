@@ -7,7 +7,7 @@ columns already resident in HBM into one JSON array, records/s; this is the
 workload the north-star target names.  The same JSON object also carries the
 flat-encode (configs[1]), skewed (configs[4]) and NDJSON-decode (configs[3])
 figures under "workloads", each with its own fraction of the HBM roofline,
-the roofline of the headline kernel measured with HIP events on the codec's
+the roofline of the headline kernel measured with the clock stamps of the codec's
 stream, and the CPU restatement timed on this host's cores.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload nested|flat|decode|skew|options]
@@ -45,7 +45,7 @@ def run_encode(codec, cols_dev, fmt, steps, warmup):
     t0 = time.perf_counter()
     for _ in range(steps):
         codec.encode(cols_dev, fmt, out=out)
-        kern.append(codec.timings()[0])      # the whole device pipeline, HIP events on the codec stream
+        kern.append(codec.timings()[0])      # the whole device pipeline, clock stamps on the codec stream
     torch.cuda.synchronize()
     wall = (time.perf_counter() - t0) / steps
     return need, wall, sum(kern) / len(kern), out
@@ -155,7 +155,7 @@ def decode_workload(codec, n, steps, warmup):
     for _ in range(steps):
         dcols, el, ec, res = codec.decode(data, out=bufs)
         # [total, fill, k_dec_lines, host gap, fill, k_dec_block, k_dec_bscan, k_dec_write, k_dec_long,
-        #  k_dec_errcode] (HIP events on the codec stream)
+        #  k_dec_errcode] (clock stamps on the codec stream)
         tm = codec.timings()
         for k, i in zip(names, (2, 5, 6, 7, 8, 9)):
             per[k].append(tm[i])
@@ -206,7 +206,7 @@ def array_decode_rates(codec, cols, caps, steps, warmup):
     t0 = time.perf_counter()
     for _ in range(steps):
         dcols, el, ec, res = codec.decode_array(doc, out=bufs)
-        kms.append(codec.timings()[0])                 # the whole pipeline, HIP events on the codec stream
+        kms.append(codec.timings()[0])                 # the whole pipeline, clock stamps on the codec stream
     torch.cuda.synchronize()
     wall = (time.perf_counter() - t0) / steps
     h = dcols.to_host()
@@ -371,7 +371,7 @@ def skew_workload(codec, n, steps, warmup, with_decode):
         t0 = time.perf_counter()
         for _ in range(dsteps):
             dcols, el, ec, res = codec.decode(text, out=bufs)
-            dev_ms.append(codec.timings()[0])    # first to last HIP event of the call
+            dev_ms.append(codec.timings()[0])    # first to last clock stamp of the call
         torch.cuda.synchronize()
         dwall = (time.perf_counter() - t0) / dsteps
         h = dcols.to_host()
@@ -441,7 +441,7 @@ def _model_bytes(cols):
 
 
 def _kernel_ms(codec, fn, steps, warmup, idx):
-    """Mean of one HIP-event interval (idx into Codec.timings()) over steps calls."""
+    """Mean of one clock-stamp interval (idx into Codec.timings()) over steps calls."""
     import torch
     for _ in range(warmup):
         fn()
