@@ -836,7 +836,7 @@ template <int MODEL> constexpr bool m_counter(int k) {
 }
 
 // Bound by the instructions of the walk (every lane its own record in LDS):
-// 1M Users (171 MB) 2.86 -> 0.27 ms, 1M Orders (123 MB) 0.77 -> 0.13 ms
+// 1M Users (171 MB) 2.86 -> 0.25 ms, 1M Orders (123 MB) 0.77 -> 0.13 ms
 // against the form that recursed from both outcomes of a property's test
 // (the User text holds escapes in one record of four and a null property in
 // more than half of them).
@@ -966,9 +966,10 @@ __device__ __forceinline__ void m_copy_esc(const MLds &L, uint32_t q, uint32_t l
 }
 
 // Bound by the scattered string stores (16-byte stores at any address).  1M
-// Users 0.61 -> 0.29 ms with the strings copied straight from the tile and
+// Users 0.61 -> 0.25 ms with the strings copied straight from the tile and
 // one exchange for all scans instead of two barriers per counter.  (Capped
-// at 168 VGPRs instead of its 232 it spills 82 and takes 0.40 ms.)
+// at 168 VGPRs instead of its 232 it spills 82: 0.40 against 0.29 ms before the
+// escapes left eight bytes at a time.)
 // ALL_TAPED: every record is on the tape (the launcher's rule), so the
 // kernel holds no reader and keeps its registers for the copies.
 template <int MODEL, int BT, int TILE, bool ALL_TAPED>
