@@ -1259,6 +1259,16 @@ pj_status index_stage(pj_ctx *ctx, const uint8_t *in, uint64_t len, bool array, 
     return fail(PJ_ERR_DEVICE, "line index did not converge");
 }
 
+// Whether every block of P.lpb lines spans less than PJ_DEC_MAX_BLOCK_SPAN.
+pj_status blocks_fit(pj_ctx *ctx, const DecParams &P, uint64_t *X, bool *fits) {
+    PJ_HIP(pj_launch_fill_u64(X + 15, 1, 0, ctx->stream));
+    PJ_HIP(pj_launch_dec_span_check(P, X + 15, ctx->stream));
+    PJ_HIP(hipMemcpyAsync(ctx->pinned, X + 15, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    PJ_HIP(hipStreamSynchronize(ctx->stream));
+    *fits = ctx->pinned[0] == 0;
+    return PJ_OK;
+}
+
 pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_columns *out, uint64_t *err_line,
                       uint8_t *err_code, uint64_t err_cap, pj_decode_result *res, bool array = false) {
     pj_status s = bind(ctx);
@@ -1273,20 +1283,6 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     uint64_t *X = nullptr, lines = 0;
     if ((s = index_stage(ctx, in, len, array, P, X, &lines))) return s;
     P.lines = lines;
-    if (len >= PJ_DEC_MAX_BLOCK_SPAN && lines) {
-        // the lines of one block must span less than 4 GiB (32-bit offsets
-        // inside a block); only an input that long can break it
-        PJ_HIP(pj_launch_fill_u64(X + 15, 1, 0, ctx->stream));
-        PJ_HIP(pj_launch_dec_span_check(P, X + 15, ctx->stream));
-        PJ_HIP(hipMemcpyAsync(ctx->pinned, X + 15, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-        PJ_HIP(hipStreamSynchronize(ctx->stream));
-        if (ctx->pinned[0]) {
-            ctx->n_ev = 0;
-            return fail(PJ_ERR_INVALID_ARG, "lines of 4 GiB or more in one block of " +
-                                                std::to_string(pj_dec_parse_block()) + " lines (offsets inside a "
-                                                "block are 32-bit)");
-        }
-    }
     P.o = *out;
     P.err_line = err_line;
     P.err_code = err_code;
@@ -1303,6 +1299,27 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     (void)hipGetLastError();
     const bool split = P.tape != nullptr;
     P.lpb = split ? pj_dec_split_block(len, lines) : pj_dec_parse_block();
+    if (len >= PJ_DEC_MAX_BLOCK_SPAN && lines) {
+        // the lines of one block must span less than 4 GiB (32-bit offsets
+        // inside a block); only an input that long can break it.  What is
+        // refused goes by the large blocks; where one of the small ones
+        // would span too much (it may lie across two large ones), the large
+        // ones are used.
+        const int want = P.lpb;
+        bool fits = false;
+        P.lpb = pj_dec_parse_block();
+        if ((s = blocks_fit(ctx, P, X, &fits))) return s;
+        if (!fits) {
+            ctx->n_ev = 0;
+            return fail(PJ_ERR_INVALID_ARG, "lines of 4 GiB or more in one block of " + std::to_string(P.lpb) +
+                                                " lines (offsets inside a block are 32-bit)");
+        }
+        if (want != P.lpb) {
+            P.lpb = want;
+            if ((s = blocks_fit(ctx, P, X, &fits))) return s;
+            if (!fits) P.lpb = pj_dec_parse_block();
+        }
+    }
     const uint64_t gp = (lines + P.lpb - 1) / P.lpb;
     // scan buffer: vector look-back words (single pass) or block totals,
     // bases and scan look-back words (split), then the deferred

@@ -3607,10 +3607,10 @@ __global__ void k_dec_span_check(const uint64_t *ls, uint64_t lines, uint64_t lp
 }  // namespace pj
 
 hipError_t pj_launch_dec_span_check(const DecParams &P, uint64_t *flag, hipStream_t st) {
-    const uint64_t nb = (P.lines + DEC_LPB - 1) / DEC_LPB;
+    const uint64_t lpb = (uint64_t)P.lpb, nb = (P.lines + lpb - 1) / lpb;
     if (!nb) return hipSuccess;
     hipLaunchKernelGGL(pj::k_dec_span_check, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, P.line_start,
-                       P.lines, (uint64_t)DEC_LPB, flag);
+                       P.lines, lpb, flag);
     return hipGetLastError();
 }
 
