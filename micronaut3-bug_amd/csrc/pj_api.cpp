@@ -39,11 +39,10 @@ pj_status fail(pj_status s, const std::string &msg) {
 struct DevBuf {
     void *p = nullptr;
     size_t n = 0;
+    uint64_t zero = 0;           // leading words known to be zero (their user keeps count); new memory: none
     hipError_t ensure(size_t want) {
         if (want <= n) return hipSuccess;
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        n = 0;
+        release();
         size_t sz = std::max<size_t>(want + want / 8, 4096);
         hipError_t e = hipMalloc(&p, sz);
         if (e == hipSuccess) n = sz;
@@ -53,6 +52,7 @@ struct DevBuf {
         if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
+        zero = 0;
     }
 };
 
@@ -99,7 +99,6 @@ struct pj_ctx {
     // Pet decodes since one with lines over the tile: while below BIG_RECENT,
     // the large-tile kernels run with the others, not in a second attempt
     int over_since = 1 << 20;
-    uint64_t scan_zero = 0;       // leading words of `scan` known to be zero (left so by the last encode)
     uint64_t *stamps = nullptr;   // MAX_EV clock stamps of the call's launches (pinned, after the 64 result words)
     double ticks_per_ms = 1e5;    // of the device's wall clock
     int n_ev = 0;
@@ -460,7 +459,6 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     const bool defer_big = nested_cols(cols) && !pretty && !count_only && !fixed_scratch;
     const uint64_t big_cap = defer_big ? std::min<uint64_t>(n, enc_big_cap()) : 0;
     uint64_t *sc;
-    const void *sc_was = ctx->scan.p;
     std::unique_lock<std::mutex> noalloc_guard;
     if (fixed_scratch) {
         if (n > PJ_NOALLOC_MAX_RECORDS(nested_cols(cols)) || nblk + 4 + 128 > PJ_NOALLOC_SCRATCH_WORDS)
@@ -473,7 +471,6 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         noalloc_guard = std::unique_lock<std::mutex>(pj::noalloc_lock(ctx->device));
     } else {
         PJ_HIP(ctx->scan.ensure((nblk + 4 + 128 + (two_pass ? GEO_WORDS * nblk : 0) + 2 * big_cap) * sizeof(uint64_t)));
-        if (sc_was != ctx->scan.p) ctx->scan_zero = 0;
         sc = static_cast<uint64_t *>(ctx->scan.p);
     }
     // the words a pass starts from zero: the last encode left them so, or a
@@ -481,8 +478,8 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     // results go out, which spares the next call the fill's launch)
     constexpr uint64_t CLEAR_AFTER = 2048;
     const uint64_t head = nblk + 4;
-    bool clean = !fixed_scratch && ctx->scan_zero >= head;
-    ctx->scan_zero = 0;
+    bool clean = !fixed_scratch && ctx->scan.zero >= head;
+    ctx->scan.zero = 0;
     // k_enc_big runs behind the pass when a recent call listed large records;
     // otherwise only once the pass's count says that there are some, after
     // the wait for it (an empty launch costs a call of a page of records 10%)
@@ -554,7 +551,7 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
             PJ_HIP(pj_launch_encode_big(P, true, ctx->stream));
             PJ_HIP(pj_launch_publish(ctx->pinned, sc, 0, 0, -1, ctx->stream, mark(ctx)));
             PJ_HIP(hipStreamSynchronize(ctx->stream));
-        } else if (!redo) ctx->scan_zero = clear;
+        } else if (!redo) ctx->scan.zero = clear;
         clean = false;
         if (!redo) break;
         P.order_by_id = 0;                                      // redo in ticket order
@@ -737,7 +734,7 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
     // (ticket, total, look-back words), the selected indices
     const uint64_t w_sel = 2 + pj_select_blocks(n), w_enc = 2 + nblk;
     PJ_HIP(ctx->scan.ensure((w_sel + w_enc + n + 1) * sizeof(uint64_t)));
-    ctx->scan_zero = 0;
+    ctx->scan.zero = 0;
     uint64_t *sc = static_cast<uint64_t *>(ctx->scan.p), *ec = sc + w_sel, *sel = ec + w_enc;
     EncParams P;
     std::memset(&P, 0, sizeof P);
@@ -1331,7 +1328,7 @@ pj_status decode_impl(pj_ctx *ctx, const uint8_t *in, uint64_t len, pj_pet_colum
     const uint64_t w_lpos = (9 * lines + 1) / 2;
     const uint64_t w_split = split ? lines + w_lpos + 2 + gp : 0;
     PJ_HIP(ctx->scan.ensure((w_state + lines + 8 + w_split) * 8));
-    ctx->scan_zero = 0;
+    ctx->scan.zero = 0;
     uint64_t *SB = static_cast<uint64_t *>(ctx->scan.p);
     P.state_parse = SB;
     P.bagg = SB;
@@ -1812,7 +1809,7 @@ extern "C" pj_status pj_encode_model_device(pj_ctx *ctx, int model, const pj_mod
     }
     const uint64_t bt = (uint64_t)pj_encode_model_records(), nblk = (n + bt - 1) / bt;
     PJ_HIP(ctx->scan.ensure((nblk + 2) * sizeof(uint64_t)));
-    ctx->scan_zero = 0;
+    ctx->scan.zero = 0;
     uint64_t *sc = static_cast<uint64_t *>(ctx->scan.p);
     ModelEncParams P;
     std::memset(&P, 0, sizeof P);
@@ -1856,7 +1853,7 @@ extern "C" pj_status pj_decode_model_device(pj_ctx *ctx, int model, const uint8_
     const uint64_t nb = (lines + pj_decode_model_block() - 1) / pj_decode_model_block();
     const uint64_t nchunks = (nb + 1023) / 1024;     // the scan's chunks of 1024 blocks
     PJ_HIP(ctx->scan.ensure((2 * nb * MD_MAXK + nchunks * MD_MAXK + MD_MAXK + 1) * sizeof(uint64_t)));
-    ctx->scan_zero = 0;
+    ctx->scan.zero = 0;
     uint64_t *SB = static_cast<uint64_t *>(ctx->scan.p);
     ModelDecParams M;
     std::memset(&M, 0, sizeof M);

@@ -3,7 +3,10 @@
 // is needed and a line of several GiB costs nothing.
 //   * decode: the line blocks that the launches get never span
 //     PJ_DEC_MAX_BLOCK_SPAN bytes, and what is refused is decided over the
-//     larger blocks whichever are used.
+//     larger blocks whichever are used;
+//   * encode: the words that a pass starts from zero are zero at its launch,
+//     also when the scratch grew in between and its new memory has the old
+//     address.
 #include <sys/mman.h>
 
 #include <cstdio>
@@ -22,7 +25,9 @@ static void expect(bool ok, const char *what, const char *where) {
 }
 
 // ------------------------------------------------------------- the runtime
-// Device memory: eight slots of address space.
+// Device memory: eight slots of address space, the lowest free one each time,
+// so that an allocation after a free has the freed address.  New memory
+// starts with other bytes than zero.
 constexpr size_t SLOT = 4ull << 30;
 constexpr int SLOTS = 8;
 static uint8_t *arena;
@@ -132,13 +137,27 @@ hipError_t pj_launch_dec_bscan(const DecParams &, hipStream_t) { return hipSucce
 hipError_t pj_launch_dec_write(const DecParams &, hipStream_t) { return hipSuccess; }
 hipError_t pj_launch_dec_long(const DecParams &, hipStream_t) { return hipSuccess; }
 hipError_t pj_launch_dec_errcode(const DecParams &, hipStream_t) { return hipSuccess; }
+// The pass: its ticket, counters and look-back words must be zero; it leaves
+// them as a pass does.
+hipError_t pj_launch_encode(const EncParams &P, bool nested, bool, hipStream_t) {
+    uint64_t *sc = reinterpret_cast<uint64_t *>(P.ticket);
+    const uint64_t nblk = (P.n + pj_encode_block_records(nested) - 1) / pj_encode_block_records(nested);
+    for (uint64_t i = 0; i < nblk + 4; i++)
+        if (sc[i]) {
+            expect(false, "a word that the pass starts from zero is not zero", where_now);
+            break;
+        }
+    sc[0] = P.order_by_id ? 0 : nblk;
+    *P.total = 100;
+    for (uint64_t i = 0; i < nblk; i++) P.state[i] = (2ull << 62) | 100;
+    return hipSuccess;
+}
 #define UNUSED_LAUNCH(name, ...) \
     hipError_t name(__VA_ARGS__) { expect(false, #name " launched", where_now); return hipSuccess; }
 UNUSED_LAUNCH(pj_launch_add_u64, uint64_t *, uint64_t, uint64_t, hipStream_t)
 UNUSED_LAUNCH(pj_launch_put_bytes, uint8_t *, uint32_t, int, hipStream_t)
 UNUSED_LAUNCH(pj_launch_copy_pieces, const CopyPieces &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_arr_frame, const DecParams &, hipStream_t)
-UNUSED_LAUNCH(pj_launch_encode, const EncParams &, bool, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_big, const EncParams &, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_rows, const EncParams &, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_pretty, const EncParams &, hipStream_t)
@@ -197,10 +216,39 @@ static void span_guard(pj_ctx *ctx) {
     unsetenv("PETJSON_DECODE_TAPE");
 }
 
+static void scratch_zero(pj_ctx *ctx) {
+    pj_pet_columns flat;
+    std::memset(&flat, 0, sizeof flat);
+    flat.id = reinterpret_cast<int64_t *>(dev);
+    flat.name_off = dev;
+    flat.name_bytes = reinterpret_cast<uint8_t *>(dev);
+    pj_pet_columns nested = flat;
+    nested.photo_off = dev;
+    nested.url_off = dev;
+    nested.url_bytes = reinterpret_cast<uint8_t *>(dev);
+    auto encode = [&](const char *what, const pj_pet_columns &from, uint64_t n) {
+        where_now = what;
+        pj_pet_columns c = from;
+        c.n_pets = n;
+        uint64_t len = 0;
+        expect(pj_encode_device(ctx, &c, PJ_FORMAT_ARRAY, reinterpret_cast<uint8_t *>(dev), sizeof dev, &len) == PJ_OK &&
+                   len == 100, "encode", what);
+    };
+    encode("flat", flat, 100000);                     // 391 blocks, the words cleared behind it
+    encode("flat again", flat, 90000);
+    encode("nested, the scratch grows for the large-record list", nested, 30000);
+    encode("nested again", nested, 20000);
+    encode("flat, past what is cleared ahead", flat, 2000000);
+    encode("flat, small", flat, 20);
+    encode("nested, grows again", nested, 900000);
+    encode("nested, small", nested, 20);
+}
+
 int main() {
     pj_status s;
     pj_ctx *ctx = pj_create(0, &s);
     if (!ctx) { std::printf("FAIL: no context\n"); return 1; }
+    scratch_zero(ctx);
     span_guard(ctx);
     pj_destroy(ctx);
     if (fails) return 1;
