@@ -3277,8 +3277,10 @@ __device__ __forceinline__ BlockCols block_cols(const pj_pet_columns &o, const u
 }
 
 // Do the call's totals fit the output capacities?  (Nothing is written
-// otherwise: the call reports PJ_ERR_CAPACITY with the sizes it needs.)
+// otherwise: the call reports PJ_ERR_CAPACITY with the sizes it needs.)  They
+// are not known before the lines over the tile are read.
 __device__ __forceinline__ bool dec_room(const DecParams &P) {
+    if (!P.big_tile && *P.over_count) return false;
     const pj_pet_columns &o = P.o;
     const uint64_t *T = P.totals;
     return T[C_PETS] <= o.cap_pets && T[C_NAMEB] <= o.cap_name_bytes && T[C_CATB] <= o.cap_cat_name_bytes &&

@@ -711,6 +711,37 @@ def test_decode_lines_around_the_tiles(codec, array):
             assert_same(gpu_decode(codec, data), orc.decode(data))
 
 
+@pytest.mark.parametrize("place", [0, 150, 299])
+def test_decode_capacity_with_a_line_over_the_tile(place):
+    """A call whose columns have room for all but its line over the tile (whose
+    size is known last) writes no record, whether that line is met for the
+    first time or a recent call had one; and with room it writes all."""
+    lines = orc.encode(pj.generate(3, 300), pj.FORMAT_NDJSON).split(b"\n")[:-1]
+    lines.insert(place, b'{"id":7,"name":"' + b"w" * 40000 + b'","photoUrls":["u"],"tags":[{"id":1,"name":"t"}]}')
+    text = b"\n".join(lines) + b"\n"
+    need = orc.decode(text)[3]
+    data = torch.frombuffer(bytearray(text), dtype=torch.uint8).cuda()
+    caps = {"cap_pets": need.n_pets, "cap_name_bytes": need.name_bytes - 1, "cap_cat_name_bytes": need.cat_name_bytes,
+            "cap_urls": need.n_urls, "cap_url_bytes": need.url_bytes, "cap_tags": need.n_tags,
+            "cap_tag_name_bytes": need.tag_name_bytes}
+    codec = pj.Codec(0)
+    try:
+        for _ in range(3):
+            dc, raw = _sentinel_columns(caps)
+            el = torch.empty(16, dtype=torch.int64, device="cuda")
+            ec = torch.empty(16, dtype=torch.uint8, device="cuda")
+            with pytest.raises(pj.PetJsonError) as ei:
+                codec.decode(data, out=(dc, el, ec))
+            assert ei.value.status == pj.PJ_ERR_CAPACITY
+            torch.cuda.synchronize()
+            for k, (b, n) in raw.items():
+                lead = 8 if k.endswith("_off") else 0        # offset arrays start with 0
+                assert not b[:lead].any() and bool((b[lead:] == 0xEE).all()), k
+            assert_same(gpu_decode(codec, text, caps={**caps, "cap_name_bytes": need.name_bytes}), orc.decode(text))
+    finally:
+        codec.close()
+
+
 @pytest.mark.parametrize("extra", [0, 40])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 103, 104, 105, 128, 129, 1000])
 def test_decode_block_sizes_by_average_line(codec, n, extra):
