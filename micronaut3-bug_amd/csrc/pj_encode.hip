@@ -2082,7 +2082,7 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
     for (uint32_t r0 = 0; r0 < live;) {
         // the run: records r0 .. r0 + k - 1 end within the tile
         const bool mine = t >= r0 && t < live && end - at <= (uint64_t)TILE;
-        if (mine && !p.count_only) {
+        if (mine) {
             LdsSinkU ls{sh.bytes, (uint32_t)(pre - at), (uint32_t)(end - at)};
             emit(ls);
         }
@@ -2097,7 +2097,6 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
             }
         }
         const uint32_t k = (uint32_t)__syncthreads_count(mine);    // (the run's tile is built, the base known)
-        if (p.count_only) return;
         const uint64_t base = sh.base;
         if (k == 0) {                        // record r0 is larger than the tile
             if (t == r0) {
@@ -2129,11 +2128,10 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
 // records, and they leave in runs through the tile.  Bound by the latency of
 // each record's reads.  A third of 2M nested records by status: 0.51 -> 0.43 ms
 // against 32-byte sectors stored by each thread; 2M flat records pretty:
-// 0.27 -> 0.16 ms.
+// 0.27 -> 0.16 ms.  Without a tile (TILE 0): the size alone.
 template <int BT, bool PRETTY, int TILE>
-__global__ __launch_bounds__(BT, 4) void k_encode_rows(EncParams P) {
+__global__ __launch_bounds__(BT, TILE ? 4 : 1) void k_encode_rows(EncParams P) {
     stamp_start(P.stamp);
-    __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
     __shared__ uint64_t sh_scan[BT / 64 + 2];
     __shared__ uint64_t sh_b;
     const ColSrc XG{P.c.name_bytes, P.c.cat_name_bytes, P.c.url_bytes, P.c.tag_name_bytes, 0, 0, 0, 0};
@@ -2156,7 +2154,13 @@ __global__ __launch_bounds__(BT, 4) void k_encode_rows(EncParams P) {
     }
     uint64_t agg;
     const uint64_t pre = block_excl_scan<BT>(cs.n, sh_scan, &agg);
-    emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
+    if constexpr (TILE > 0) {
+        __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
+        emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
+    } else if (t < 64) {
+        const uint64_t excl = lookback(P.state, b, agg);
+        if (t == 0 && b == nblk - 1) *P.total = excl + agg;
+    }
 }
 
 // The records whose status code is in the mask (bit s: status s, bit 3: no
@@ -2552,6 +2556,11 @@ hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t st) {
 // runs per block) 0.522 / 0.180.
 constexpr int ENC_PRETTY_BT = 256, ENC_ROWS_TILE = 39 * 1024;
 int pj_encode_pretty_records() { return ENC_PRETTY_BT; }
+// The size alone holds no tile and is bound by the look-backs that the blocks
+// chain: 512 records per block, 2M flat / 1M nested records 0.096 / 0.188 ms
+// per call, against 0.150 / 0.224 with 256.
+constexpr int ENC_SIZE_BT = 512;
+int pj_encode_pretty_size_records() { return ENC_SIZE_BT; }
 
 constexpr int ENC_SEL_BT = 256, ENC_SEL_R = 16;
 
@@ -2567,6 +2576,12 @@ hipError_t pj_launch_encode_rows(const EncParams &P, bool pretty, hipStream_t st
 }
 
 uint64_t pj_select_blocks(uint64_t n) { return (n + ENC_SEL_BT * ENC_SEL_R - 1) / (ENC_SEL_BT * ENC_SEL_R); }
+
+hipError_t pj_launch_pretty_size(const EncParams &P, hipStream_t st) {
+    const uint64_t nblk = (P.n + ENC_SIZE_BT - 1) / ENC_SIZE_BT;
+    hipLaunchKernelGGL((pj::k_encode_rows<ENC_SIZE_BT, true, 0>), dim3((unsigned)nblk), dim3(ENC_SIZE_BT), 0, st, P);
+    return hipGetLastError();
+}
 
 hipError_t pj_launch_select_status(const EncParams &P, uint32_t mask, uint64_t *sel, hipStream_t st) {
     hipLaunchKernelGGL((pj::k_select_status<ENC_SEL_BT, ENC_SEL_R>), dim3((unsigned)pj_select_blocks(P.c.n_pets)),

@@ -94,6 +94,7 @@ int pj_decode_model_block() { return 128; }
 int pj_encode_block_records(bool nested) { return nested ? 96 : 256; }
 int pj_encode_model_records() { return 512; }
 int pj_encode_pretty_records() { return 256; }
+int pj_encode_pretty_size_records() { return 512; }
 int pj_encode_pretty_tile_records() { return 64; }
 uint64_t pj_select_blocks(uint64_t n) { return (n + 4095) / 4096; }
 hipError_t pj_noalloc_scratch_init(int, uint64_t **p) { *p = nullptr; return hipSuccess; }
@@ -160,6 +161,7 @@ UNUSED_LAUNCH(pj_launch_copy_pieces, const CopyPieces &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_arr_frame, const DecParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_big, const EncParams &, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_rows, const EncParams &, bool, hipStream_t)
+UNUSED_LAUNCH(pj_launch_pretty_size, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_pretty, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_measure, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_model, const ModelEncParams &, hipStream_t)

@@ -618,3 +618,13 @@ def test_encode_scratch_left_clear_between_calls(codec):
         enc(small)
     enc(skew)
     enc(skew)
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 511, 512, 513, 1025, 70_000])
+def test_encode_pretty_size_around_its_blocks(codec, n):
+    """The pretty size alone (blocks of 512 records): around the edges of its
+    blocks and of the writer's, over more blocks than one look-back step
+    reads, flat and nested."""
+    for config in (2, 3):
+        cols = pj.generate(config, n, seed=n)
+        assert codec.encode_size(cols.to_device(), pj.FORMAT_PRETTY) == len(orc.encode(cols, pj.FORMAT_PRETTY))
