@@ -2064,9 +2064,18 @@ __global__ __launch_bounds__(BT) void k_enc_measure(EncParams P) {
 // of `live`, n bytes long; pre is its offset in the block and agg the block's
 // length.  Runs of records that fit the LDS tile are built there (emit(sink),
 // LdsSinkU) and leave with aligned 16-byte stores (tile_copy_out), the first
-// run while the look-back resolves; a record larger than the tile is written
-// by its own thread (SectorSink).  Bytes past the capacity are not written;
+// run while the look-back resolves.  Bytes past the capacity are not written;
 // the last block stores the total.  All threads call.
+//
+// A run's records are built while the rest of the block waits.  A block whose
+// tile holds less than a quarter of its records on average, or with a record
+// over the tile, is therefore written by all its threads at once (SectorSink).
+// By runs / by threads, us per call, flat Pets selected (256 records, 39 KiB)
+// of 520 bytes 272 / 292, 670: 337 / 269, 1,070: 637 / 295, 10 KB: 25,400 / 1,895;
+// Users (512 records, 78 KiB) of 412 bytes 194 / 190, 712: 264 / 271, 892:
+// 401 / 333, 1,912: 1,390 / 636, 24 KB: 130,000 / 7,490; 250,000 skewed Pets
+// selected 11,000 / 6,950, and 7,040 with this rule (the line at a sixth:
+// 9,500, at a third: 7,200).
 template <int BT, int TILE> struct RunTile {
     uint8_t bytes[TILE + 32];                    // tile_copy_out reads 32 bytes past
     uint64_t base, end;
@@ -2077,46 +2086,43 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
     const uint32_t t = threadIdx.x;
     const uint64_t end = pre + n;
     if (t == 0) lb_publish(p.state, b, agg);
-    bool placed = false;                     // sh.base holds the block's offset
+    auto place = [&] {                       // the block's offset, by its first wave
+        if (t < 64) {
+            const uint64_t excl = lb_resolve(p.state, b, agg);
+            if (t == 0) {
+                sh.base = excl;
+                if (b == nblk - 1) *p.total = excl + agg;
+            }
+        }
+    };
+    constexpr uint64_t AVG = 4 * TILE / BT;  // average record above which the threads write
+    if (__syncthreads_or(agg > AVG * live || n > (uint64_t)TILE)) {
+        place();
+        __syncthreads();
+        if (t < live && sh.base + end <= p.cap) {
+            SectorSink xs;
+            xs.init(p.out + sh.base + pre);
+            emit(xs);
+            xs.finish();
+        }
+        return;
+    }
     uint64_t at = 0;                         // block offset of the run's first record
     for (uint32_t r0 = 0; r0 < live;) {
-        // the run: records r0 .. r0 + k - 1 end within the tile
+        // the run: records r0 .. r0 + k - 1 end within the tile (k > 0: each fits it)
         const bool mine = t >= r0 && t < live && end - at <= (uint64_t)TILE;
         if (mine) {
             LdsSinkU ls{sh.bytes, (uint32_t)(pre - at), (uint32_t)(end - at)};
             emit(ls);
         }
-        if (!placed) {
-            placed = true;
-            if (t < 64) {
-                const uint64_t excl = lb_resolve(p.state, b, agg);
-                if (t == 0) {
-                    sh.base = excl;
-                    if (b == nblk - 1) *p.total = excl + agg;
-                }
-            }
-        }
+        if (r0 == 0) place();
         const uint32_t k = (uint32_t)__syncthreads_count(mine);    // (the run's tile is built, the base known)
-        const uint64_t base = sh.base;
-        if (k == 0) {                        // record r0 is larger than the tile
-            if (t == r0) {
-                if (base + end <= p.cap) {
-                    SectorSink xs;
-                    xs.init(p.out + base + pre);
-                    emit(xs);
-                    xs.finish();
-                }
-                sh.end = end;
-            }
-        } else if (t == r0 + k - 1) sh.end = end;
+        if (t == r0 + k - 1) sh.end = end;
         __syncthreads();
-        const uint64_t stop = sh.end;
-        if (k) {
-            const uint64_t hi = min(base + stop, p.cap);
-            if (base + at < hi) tile_copy_out<BT>(sh.bytes, p.out, base + at, base + at, hi, t);
-        }
+        const uint64_t stop = sh.end, base = sh.base, hi = min(base + stop, p.cap);
+        if (base + at < hi) tile_copy_out<BT>(sh.bytes, p.out, base + at, base + at, hi, t);
         at = stop;
-        r0 += k ? k : 1;
+        r0 += k;
         __syncthreads();                     // the tile and sh.end are free for the next run
     }
 }
@@ -2125,8 +2131,8 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
 // pretty-printed output (PRETTY), and the records a selection names
 // (P.sel: output record j is column record sel[j]; compact or pretty).  Each
 // thread measures its record from global memory, a block scan places the
-// records, and they leave in runs through the tile.  Bound by the latency of
-// each record's reads.  A third of 2M nested records by status: 0.51 -> 0.43 ms
+// records, and they leave in runs through the tile (emit_runs).  Bound by the
+// latency of each record's reads.  A third of 2M nested records by status: 0.51 -> 0.43 ms
 // against 32-byte sectors stored by each thread; 2M flat records pretty:
 // 0.27 -> 0.16 ms.  Without a tile (TILE 0): the size alone.
 template <int BT, bool PRETTY, int TILE>
@@ -2550,7 +2556,7 @@ hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t st) {
     return hipGetLastError();
 }
 
-// 256-record blocks with a 39 KiB tile, four workgroups per CU.  A third of 2M
+// 256-record blocks with a 39 KiB tile, four workgroups per CU (all by runs).  A third of 2M
 // nested records / 2M flat records pretty: 0.428 / 0.163 ms; 512 records and
 // 78 KiB 0.437 / 0.152, 128 and 19 KiB 0.431 / 0.232, 512 and 52 KiB (three
 // runs per block) 0.522 / 0.180.

@@ -628,3 +628,48 @@ def test_encode_pretty_size_around_its_blocks(codec, n):
     for config in (2, 3):
         cols = pj.generate(config, n, seed=n)
         assert codec.encode_size(cols.to_device(), pj.FORMAT_PRETTY) == len(orc.encode(cols, pj.FORMAT_PRETTY))
+
+
+@pytest.mark.parametrize("fmt", [pj.FORMAT_ARRAY, pj.FORMAT_NDJSON, pj.FORMAT_PRETTY])
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 600])
+def test_row_encode_runs_match_oracle(codec, n, fmt):
+    """Selected and pretty records leave in blocks of 256, in runs of whole
+    records through a tile of 39,936 bytes, or by their own threads where they
+    average over 624 bytes or one is over the tile: blocks of one run and of
+    several, averages on both sides of the line, a record that fills the tile
+    to the byte, is one byte longer or larger (first, last, in between), and the
+    output cut at and inside the runs."""
+    rng = np.random.default_rng(n)
+    # each record's bytes without its name
+    bare = _with_names(pj.generate(2, n, seed=n), np.zeros(1, int), rng, 0.0)
+    frame = np.array([len(x) + 1 for x in orc.encode(bare, pj.FORMAT_NDJSON).split(b"\n")[:-1]])
+    if fmt == pj.FORMAT_PRETTY:
+        frame += (len(orc.encode(bare, fmt)) - frame.sum()) // n
+    for mean in (10, 100, 530, 534, 538, 542, 546, 550, 560, 900, 3000):
+        lens = np.full(n, mean) if 530 <= mean <= 560 else rng.integers(mean // 2, mean + mean // 2 + 1, n)
+        if mean == 100:
+            for k, size in ((0, 39_936), (n - 1, 60_000), (n // 2, 39_937), (n // 3, 39_935)):
+                lens[k] = size - frame[k]
+        cols = _with_names(pj.generate(2, n, seed=n), lens, rng, 0.0 if mean == 100 else 0.02)
+        dev = cols.to_device()
+        want, wm = orc.encode_by_status(cols, 15, fmt)
+        assert wm == n
+        out = torch.full((len(want) + 64,), 0xEE, dtype=torch.uint8, device="cuda")
+        got, m = codec.encode_by_status(dev, 15, fmt, out=out)
+        assert m == n and got.cpu().numpy().tobytes() == want, mean
+        assert bool((out[len(want):] == 0xEE).all())
+        some, sm = orc.encode_by_status(cols, 0b010, fmt)
+        got, m = codec.encode_by_status(dev, 0b010, fmt, out=out)
+        assert m == sm and got.cpu().numpy().tobytes() == some, mean
+        if fmt == pj.FORMAT_PRETTY:
+            out.fill_(0xEE)
+            assert codec.encode(dev, fmt, out=out).cpu().numpy().tobytes() == want, mean
+        for cap in {len(want) - 1, len(want) // 2, 1} - {0}:
+            out.fill_(0xEE)
+            with pytest.raises(pj.PetJsonError) as ei:
+                codec.encode_by_status(dev, 15, fmt, out=out[:cap])
+            assert ei.value.status == pj.PJ_ERR_CAPACITY
+            host = out.cpu().numpy()
+            assert (host[cap:] == 0xEE).all()
+            w = host[:cap] != 0xEE
+            assert (host[:cap][w] == np.frombuffer(want, np.uint8)[:cap][w]).all()
