@@ -93,9 +93,11 @@ struct pj_ctx {
     hipEvent_t seg_done[2] = {};      // streamed encode: a segment's bytes and length are final
     uint64_t *noalloc_scratch = nullptr;  // this device's fixed encode scratch (device address)
     bool flat_wide = false;       // flat encodes use the wide tile (records seen too long for the compact one)
-    // nested encodes since one listed large records: while below BIG_RECENT,
-    // k_enc_big follows the pass without waiting for its count
-    int big_since = 1 << 20;
+    // nested encodes since one listed large records (-1: none has run): from 0
+    // to below BIG_RECENT, k_enc_big follows the pass without waiting for its
+    // count; where it must (segments, two passes), it gets a full grid below
+    // BIG_RECENT
+    int big_since = -1;
     // Pet decodes since one with lines over the tile: while below BIG_RECENT,
     // the large-tile kernels run with the others, not in a second attempt
     int over_since = 1 << 20;
@@ -484,7 +486,8 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     // k_enc_big runs behind the pass when a recent call listed large records;
     // otherwise only once the pass's count says that there are some, after
     // the wait for it (an empty launch costs a call of a page of records 10%)
-    const bool big_now = big_cap && (seg || two_pass || ctx->big_since < BIG_RECENT);
+    const bool big_recent = ctx->big_since < BIG_RECENT;
+    const bool big_now = big_cap && (seg || two_pass || (big_recent && ctx->big_since >= 0));
     EncParams P;
     std::memset(&P, 0, sizeof P);
     P.c = *cols;
@@ -531,11 +534,11 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
                 P.stamp = nullptr;
                 P.geo = geo;
                 PJ_HIP(pj_launch_encode(P, true, false, ctx->stream));
-                if (big_now) PJ_HIP(pj_launch_encode_big(P, ctx->big_since < BIG_RECENT, ctx->stream));
+                if (big_now) PJ_HIP(pj_launch_encode_big(P, big_recent, ctx->stream));
             }
         } else {
             PJ_HIP(pj_launch_encode(P, nested_cols(cols), ctx->flat_wide, ctx->stream));
-            if (big_now) PJ_HIP(pj_launch_encode_big(P, ctx->big_since < BIG_RECENT, ctx->stream));
+            if (big_now) PJ_HIP(pj_launch_encode_big(P, big_recent, ctx->stream));
         }
         if (seg) {
             PJ_HIP(hipMemcpyAsync(seg->len, sc + 1, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -559,7 +562,7 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         P.order_by_id = 0;                                      // redo in ticket order
         ctx->n_ev = 0;
     }
-    if (big_cap) ctx->big_since = ctx->pinned[3] ? 0 : std::min(ctx->big_since + 1, 1 << 20);
+    if (big_cap) ctx->big_since = ctx->pinned[3] ? 0 : ctx->big_since < 0 ? BIG_RECENT : std::min(ctx->big_since + 1, 1 << 20);
     // flat records too long for the compact tile: later calls use the wide one
     if (!pretty && !nested_cols(cols) && !ctx->flat_wide && ctx->pinned[2] * 64 > nblk) ctx->flat_wide = true;
     finish_timing(ctx);

@@ -6,7 +6,7 @@
 //     larger blocks whichever are used;
 //   * encode: the words that a pass starts from zero are zero at its launch,
 //     also when the scratch grew in between and its new memory has the old
-//     address.
+//     address; large records get a full grid where their count is not known.
 #include <sys/mman.h>
 
 #include <cstdio>
@@ -138,32 +138,39 @@ hipError_t pj_launch_dec_bscan(const DecParams &, hipStream_t) { return hipSucce
 hipError_t pj_launch_dec_write(const DecParams &, hipStream_t) { return hipSuccess; }
 hipError_t pj_launch_dec_long(const DecParams &, hipStream_t) { return hipSuccess; }
 hipError_t pj_launch_dec_errcode(const DecParams &, hipStream_t) { return hipSuccess; }
+
+static uint64_t large_records;           // that the pass lists
 // The pass: its ticket, counters and look-back words must be zero; it leaves
 // them as a pass does.
 hipError_t pj_launch_encode(const EncParams &P, bool nested, bool, hipStream_t) {
     uint64_t *sc = reinterpret_cast<uint64_t *>(P.ticket);
     const uint64_t nblk = (P.n + pj_encode_block_records(nested) - 1) / pj_encode_block_records(nested);
-    for (uint64_t i = 0; i < nblk + 4; i++)
+    for (uint64_t i = 0; i < nblk + 4 && !P.geo; i++)
         if (sc[i]) {
             expect(false, "a word that the pass starts from zero is not zero", where_now);
             break;
         }
     sc[0] = P.order_by_id ? 0 : nblk;
     *P.total = 100;
+    if (P.big_cap) *P.big_count = large_records;
     for (uint64_t i = 0; i < nblk; i++) P.state[i] = (2ull << 62) | 100;
     return hipSuccess;
 }
+static std::vector<bool> big_grids;      // full or not, of each launch for the large records
+hipError_t pj_launch_encode_big(const EncParams &, bool full, hipStream_t) {
+    big_grids.push_back(full);
+    return hipSuccess;
+}
+hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t) { *P.ticket = 1; return hipSuccess; }
 #define UNUSED_LAUNCH(name, ...) \
     hipError_t name(__VA_ARGS__) { expect(false, #name " launched", where_now); return hipSuccess; }
 UNUSED_LAUNCH(pj_launch_add_u64, uint64_t *, uint64_t, uint64_t, hipStream_t)
 UNUSED_LAUNCH(pj_launch_put_bytes, uint8_t *, uint32_t, int, hipStream_t)
 UNUSED_LAUNCH(pj_launch_copy_pieces, const CopyPieces &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_arr_frame, const DecParams &, hipStream_t)
-UNUSED_LAUNCH(pj_launch_encode_big, const EncParams &, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_rows, const EncParams &, bool, hipStream_t)
 UNUSED_LAUNCH(pj_launch_pretty_size, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_pretty, const EncParams &, hipStream_t)
-UNUSED_LAUNCH(pj_launch_encode_measure, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_model, const ModelEncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_decode_model, const ModelDecParams &, int, hipStream_t)
 UNUSED_LAUNCH(pj_launch_select_status, const EncParams &, uint32_t, uint64_t *, hipStream_t)
@@ -246,7 +253,46 @@ static void scratch_zero(pj_ctx *ctx) {
     encode("nested, small", nested, 20);
 }
 
+// Large records that the pass lists are written behind it.  Where its count
+// is not waited for, their launch has a full grid unless the last nested
+// encode is known to have listed none.
+static void large_record_launches() {
+    pj_status st;
+    pj_ctx *ctx = pj_create(0, &st);
+    pj_pet_columns c;
+    std::memset(&c, 0, sizeof c);
+    c.n_pets = 1000;
+    c.id = reinterpret_cast<int64_t *>(dev);
+    c.name_off = c.photo_off = c.url_off = dev;
+    c.name_bytes = c.url_bytes = reinterpret_cast<uint8_t *>(dev);
+    auto encode = [&](const char *what, uint64_t large, bool two_pass, std::vector<bool> want) {
+        where_now = what;
+        large_records = large;
+        big_grids.clear();
+        if (two_pass) setenv("PETJSON_ENC_TWO_PASS", "1", 1);
+        uint64_t len = 0;
+        expect(pj_encode_device(ctx, &c, PJ_FORMAT_ARRAY, reinterpret_cast<uint8_t *>(dev), sizeof dev, &len) == PJ_OK,
+               "encode", what);
+        unsetenv("PETJSON_ENC_TWO_PASS");
+        expect(big_grids == want, "launches for large records", what);
+    };
+    encode("two passes, the context's first call", 9, true, {true});
+    pj_destroy(ctx);
+    ctx = pj_create(0, &st);
+    encode("one pass, none listed", 0, false, {});
+    encode("two passes after none", 0, true, {false});
+    encode("one pass, the first large records", 9, false, {true});
+    encode("one pass after some", 0, false, {true});
+    encode("two passes after some", 9, true, {true});
+    for (int k = 0; k < 15; k++) encode("recent", 0, false, {true});
+    encode("no longer recent", 0, false, {true});
+    encode("none for long", 0, false, {});
+    large_records = 0;
+    pj_destroy(ctx);
+}
+
 int main() {
+    large_record_launches();
     pj_status s;
     pj_ctx *ctx = pj_create(0, &s);
     if (!ctx) { std::printf("FAIL: no context\n"); return 1; }
