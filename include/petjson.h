@@ -255,7 +255,8 @@ pj_status pj_encode_device_noalloc(pj_ctx *ctx, const pj_pet_columns *cols, int 
 /* Pinned (page-locked) host memory for the *_host entry points.  Inputs and
  * outputs that lie in it move by DMA straight between the caller's buffer
  * and the device; other host memory is copied through the library's pinned
- * bounce buffers first.  No counterpart in the reference; it is for callers
+ * bounce buffers first, as are all inputs and outputs of host decodes up to
+ * 4 MiB.  No counterpart in the reference; it is for callers
  * that stage their bytes in memory they allocate once (a Java caller would
  * wrap it in a MemorySegment).  Returns NULL when the allocation fails. */
 void       *pj_host_alloc(uint64_t n);

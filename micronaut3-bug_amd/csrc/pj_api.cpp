@@ -282,13 +282,15 @@ pj_status d2h(pj_ctx *c, void *host, const void *dev, size_t n, hipEvent_t after
     return PJ_OK;
 }
 
-// Copies of at most SMALL_COPY bytes in all (SMALL_PINNED when the host side is
-// pinned, whose own DMA needs no bounce copy) go through the bounce buffers in
+// Copies of at most SMALL_COPY bytes in all go through the bounce buffers in
 // one launch on the context stream, 16 bytes per access straight from or to
 // the pinned memory: for a few pieces of a few KiB the copy calls, each with
-// its events and its wait, cost far more than the bytes (decode of a body of
-// 20 records, 17 columns out: 0.76 ms with them, 0.14 ms now).
-constexpr size_t SMALL_COPY = 4 << 20, SMALL_PINNED = 64 << 10;
+// its events and its wait, cost far more than the bytes.  Array bodies decoded
+// host to host (17 columns out), copy calls / one launch: 5 KiB 730 / 127 us,
+// 1 MiB 890 / 210, 3.8 MiB 1,090 / 400; pinned by the caller (no bounce copy in
+// the copy calls) 400 / 126, 400 / 205, 510 / 402, and from 6.4 MiB no better
+// (575 / 587; 10 MiB 710 / 870).
+constexpr size_t SMALL_COPY = 4 << 20;
 struct Piece {
     void *dst;
     const void *src;
@@ -302,8 +304,7 @@ pj_status h2d_input(pj_ctx *c, void *dev, const void *host, size_t n) {
     if (!n) return PJ_OK;
     pj_status s = xfer_init(c->xin);
     if (s) return s;
-    if (n > std::min(SMALL_COPY, c->xin.chunk & ~size_t(15)) || (n > SMALL_PINNED && pinned_host(host, n)))
-        return h2d(c, dev, host, n);
+    if (n > std::min(SMALL_COPY, c->xin.chunk & ~size_t(15))) return h2d(c, dev, host, n);
     std::memcpy(c->xin.bounce[0], host, n);
     CopyPieces C{};
     C.dst[0] = static_cast<uint8_t *>(dev);
@@ -320,13 +321,8 @@ pj_status d2h_pieces(pj_ctx *c, const Piece *p, int k) {
     pj_status s = xfer_init(c->xout);
     if (s) return s;
     uint64_t total = 0;
-    int big = 0;                             // the largest piece stands for all of them
-    for (int j = 0; j < k; j++) {
-        total += align16(p[j].n);
-        if (p[j].n > p[big].n) big = j;
-    }
-    if (total > std::min(SMALL_COPY, c->xout.chunk) || k > 20 ||
-        (total > SMALL_PINNED && pinned_host(p[big].dst, p[big].n))) {
+    for (int j = 0; j < k; j++) total += align16(p[j].n);
+    if (total > std::min(SMALL_COPY, c->xout.chunk) || k > 20) {
         for (int j = 0; j < k; j++)
             if (p[j].n && (s = d2h(c, p[j].dst, p[j].src, p[j].n, nullptr, false))) return s;
         return d2h_wait(c);
@@ -477,8 +473,11 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         sc = static_cast<uint64_t *>(ctx->scan.p);
     }
     // the words a pass starts from zero: the last encode left them so, or a
-    // fill clears them (up to CLEAR_AFTER of them are cleared again as the
-    // results go out, which spares the next call the fill's launch)
+    // fill clears them.  Up to CLEAR_AFTER of them are cleared again as the
+    // results go out, by the one workgroup that publishes these, which spares
+    // the next call the fill's launch: 31.7 -> 29.0 us for 20 flat records, 54.0
+    // -> 51.5 for 520,000 (2,036 words); the gain fades with the words to clear
+    // (7,800 of them: 114.0 -> 112.6).
     constexpr uint64_t CLEAR_AFTER = 2048;
     const uint64_t head = nblk + 4;
     bool clean = !fixed_scratch && ctx->scan.zero >= head;

@@ -283,7 +283,7 @@ import numpy as np
 import petjson as pj, oracle_py as orc
 codec = pj.Codec(0)
 # column bytes from a few KiB to past 4 MiB (one launch to the bounce buffer
-# below, the copy engine above), pinned outputs past 64 KiB
+# below, the copy engine above), in ordinary and in pinned memory
 for n in (0, 1, 3, 150, 400, 11000, 14000, 16000, 20000):
     text = np.frombuffer(orc.encode(pj.generate(3, n), pj.FORMAT_NDJSON) + b'{"name":1}\n{"name":"x","photoUrls":[]}', np.uint8)
     ref, rel, rec, rres = orc.decode(text.tobytes())
@@ -325,8 +325,8 @@ print("small copies ok")
 @pytest.mark.parametrize("chunk", [0, 4096, 100_000])
 def test_host_decode_small_copies(chunk):
     """Host decodes whose bytes go through the bounce buffers in one launch,
-    and those on the other side of that rule (by size, by pinned memory, by
-    the bounce buffers' own size), against the oracle; nothing is written past
+    and those on the other side of that rule (by size, by the bounce buffers'
+    own size), from and to ordinary and pinned memory, against the oracle; nothing is written past
     a column's end."""
     env = dict(os.environ, PYTHONPATH=os.pathsep.join([os.path.join(ROOT, "micronaut3-bug_amd"), os.path.join(ROOT, "tests")]))
     if chunk:
