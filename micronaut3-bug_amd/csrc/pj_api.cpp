@@ -439,10 +439,11 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
     // at 10M records), and the fixed scratch, sized for blocks of 96, keeps
     // that kernel too
     const bool pretty_tiled = pretty && nested_cols(cols) && !fixed_scratch && !count_only;
-    const uint64_t bt = (uint64_t)(pretty_tiled           ? pj_encode_pretty_tile_records()
-                                   : pretty && count_only ? pj_encode_pretty_size_records()
-                                   : pretty               ? pj_encode_pretty_records()
-                                                          : pj_encode_block_records(nested_cols(cols)));
+    const bool rows_size = pretty && !pretty_tiled && (count_only || !cap);
+    const uint64_t bt = (uint64_t)(pretty_tiled ? pj_encode_pretty_tile_records()
+                                   : rows_size  ? pj_encode_rows_size_records()
+                                   : pretty     ? pj_encode_pretty_records()
+                                                : pj_encode_block_records(nested_cols(cols)));
     const uint64_t nblk = (n + bt - 1) / bt;
     // Nested records: the size alone comes from the measuring pass
     // (k_enc_measure), which also gives every block its bounds and offset.
@@ -523,7 +524,7 @@ pj_status encode_impl(pj_ctx *ctx, const pj_pet_columns *cols, int format, uint8
         if (!clean) PJ_HIP(pj_launch_fill_u64(sc, head, 0, ctx->stream, t0));
         P.stamp = t1;
         if (pretty_tiled) PJ_HIP(pj_launch_encode_pretty(P, ctx->stream));
-        else if (pretty && count_only) PJ_HIP(pj_launch_pretty_size(P, ctx->stream));
+        else if (rows_size) PJ_HIP(pj_launch_rows_size(P, true, ctx->stream));
         else if (pretty) PJ_HIP(pj_launch_encode_rows(P, true, ctx->stream));
         else if (two_pass) {
             P.geo = geo;
@@ -780,7 +781,9 @@ pj_status pj_encode_by_status_device(pj_ctx *ctx, const pj_pet_columns *cols, ui
     P.ticket = reinterpret_cast<unsigned long long *>(ec);
     P.total = ec + 1;
     P.state = ec + 2;
-    PJ_HIP(pj_launch_encode_rows(P, format == PJ_FORMAT_PRETTY, ctx->stream));
+    // (without room the call only asks for the size)
+    if (out_cap) PJ_HIP(pj_launch_encode_rows(P, format == PJ_FORMAT_PRETTY, ctx->stream));
+    else PJ_HIP(pj_launch_rows_size(P, format == PJ_FORMAT_PRETTY, ctx->stream));
     PJ_HIP(pj_launch_publish(ctx->pinned, ec + 1, 1, 0, -1, ctx->stream, mark(ctx)));
     PJ_HIP(hipStreamSynchronize(ctx->stream));
     finish_timing(ctx);

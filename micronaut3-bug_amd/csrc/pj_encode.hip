@@ -2318,14 +2318,14 @@ __device__ __forceinline__ void m_rec(S &s, const ModelEncParams &P, uint64_t i,
 
 // One thread per record in blocks of BT claimed by ticket: the values are
 // loaded once, measured, placed by a block scan and written in runs through
-// the tile.  Bound by the instructions of the two passes over each record and
-// by the latency of its scattered string reads.  1M Orders (178 MB moved)
-// 0.189 -> 0.103 ms and 1M Users 0.344 -> 0.237 ms against a second pass that
-// loaded the values again and stored 32-byte sectors from each thread.
+// the tile (TILE 0: the size alone).  Bound by the instructions of the two
+// passes over each record and by the latency of its scattered string reads.
+// 1M Orders (178 MB moved) 0.189 -> 0.103 ms and 1M Users 0.344 -> 0.237 ms
+// against a second pass that loaded the values again and stored 32-byte
+// sectors from each thread.
 template <int MODEL, bool PRETTY, int BT, int TILE>
-__global__ __launch_bounds__(BT, 4) void k_encode_model(ModelEncParams P) {
+__global__ __launch_bounds__(BT, TILE ? 4 : 1) void k_encode_model(ModelEncParams P) {
     stamp_start(P.stamp);
-    __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
     __shared__ uint64_t sh_scan[BT / 64 + 2];
     __shared__ uint64_t sh_b;
     const uint32_t t = threadIdx.x;
@@ -2343,7 +2343,13 @@ __global__ __launch_bounds__(BT, 4) void k_encode_model(ModelEncParams P) {
     }
     uint64_t agg;
     const uint64_t pre = block_excl_scan<BT>(cs.n, sh_scan, &agg);
-    emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
+    if constexpr (TILE > 0) {
+        __shared__ __attribute__((aligned(16))) RunTile<BT, TILE> run;
+        emit_runs<BT, TILE>(P, run, b, nblk, live, pre, cs.n, agg, emit);
+    } else if (t < 64) {
+        const uint64_t excl = lookback(P.state, b, agg);
+        if (t == 0 && b == nblk - 1) *P.total = excl + agg;
+    }
 }
 
 __global__ void k_add_u64(uint64_t *p, uint64_t n, uint64_t v) {
@@ -2562,11 +2568,13 @@ hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t st) {
 // runs per block) 0.522 / 0.180.
 constexpr int ENC_PRETTY_BT = 256, ENC_ROWS_TILE = 39 * 1024;
 int pj_encode_pretty_records() { return ENC_PRETTY_BT; }
-// The size alone holds no tile and is bound by the look-backs that the blocks
-// chain: 512 records per block, 2M flat / 1M nested records 0.096 / 0.188 ms
-// per call, against 0.150 / 0.224 with 256.
+// The size alone (also that of a call without room for output) holds no tile
+// and is bound by the look-backs that the blocks chain: 512 records per block,
+// 2M flat / 1M nested records 0.096 / 0.188 ms per call, against 0.150 / 0.224
+// with 256.  A third of 2M nested records by status 0.23 ms, against 0.42 with the
+// writer's kernel, which builds every run before it finds no room.
 constexpr int ENC_SIZE_BT = 512;
-int pj_encode_pretty_size_records() { return ENC_SIZE_BT; }
+int pj_encode_rows_size_records() { return ENC_SIZE_BT; }
 
 constexpr int ENC_SEL_BT = 256, ENC_SEL_R = 16;
 
@@ -2583,9 +2591,10 @@ hipError_t pj_launch_encode_rows(const EncParams &P, bool pretty, hipStream_t st
 
 uint64_t pj_select_blocks(uint64_t n) { return (n + ENC_SEL_BT * ENC_SEL_R - 1) / (ENC_SEL_BT * ENC_SEL_R); }
 
-hipError_t pj_launch_pretty_size(const EncParams &P, hipStream_t st) {
+hipError_t pj_launch_rows_size(const EncParams &P, bool pretty, hipStream_t st) {
     const uint64_t nblk = (P.n + ENC_SIZE_BT - 1) / ENC_SIZE_BT;
-    hipLaunchKernelGGL((pj::k_encode_rows<ENC_SIZE_BT, true, 0>), dim3((unsigned)nblk), dim3(ENC_SIZE_BT), 0, st, P);
+    hipLaunchKernelGGL((pretty ? pj::k_encode_rows<ENC_SIZE_BT, true, 0> : pj::k_encode_rows<ENC_SIZE_BT, false, 0>),
+                       dim3((unsigned)nblk), dim3(ENC_SIZE_BT), 0, st, P);
     return hipGetLastError();
 }
 
@@ -2599,18 +2608,26 @@ hipError_t pj_launch_select_status(const EncParams &P, uint32_t mask, uint64_t *
 // workgroups.  1M Orders 0.103 ms, 1M Users 0.237 ms; 256 records and 39 KiB
 // 0.107 / 0.237, 256 and 31 KiB 0.112 / 0.262, 128 and 19 KiB 0.130 / 0.236
 // (more look-backs chained), 256 and 39 KiB without the 128-VGPR cap that
-// four waves per SIMD need 0.108 / 0.256.
+// four waves per SIMD need 0.108 / 0.256.  A call without room for output asks
+// for the size: no tile, nothing built (1M Orders / Users 63 / 92 us per call,
+// 92 / 209 with the writer).
 constexpr int ENC_MODEL_BT = 512, ENC_MODEL_TILE = 78 * 1024;
 int pj_encode_model_records() { return ENC_MODEL_BT; }
 
+namespace {
+template <int MODEL> auto model_kernel(bool pretty, bool size) {
+    return pretty ? size ? pj::k_encode_model<MODEL, true, ENC_MODEL_BT, 0>
+                         : pj::k_encode_model<MODEL, true, ENC_MODEL_BT, ENC_MODEL_TILE>
+                  : size ? pj::k_encode_model<MODEL, false, ENC_MODEL_BT, 0>
+                         : pj::k_encode_model<MODEL, false, ENC_MODEL_BT, ENC_MODEL_TILE>;
+}
+}  // namespace
+
 hipError_t pj_launch_encode_model(const ModelEncParams &P, hipStream_t st) {
     const uint64_t nblk = (P.n + ENC_MODEL_BT - 1) / ENC_MODEL_BT;
-    const bool pretty = P.format == PJ_FORMAT_PRETTY;
-    const auto kern = P.model == PJ_MODEL_ORDER
-                          ? (pretty ? pj::k_encode_model<PJ_MODEL_ORDER, true, ENC_MODEL_BT, ENC_MODEL_TILE>
-                                    : pj::k_encode_model<PJ_MODEL_ORDER, false, ENC_MODEL_BT, ENC_MODEL_TILE>)
-                          : (pretty ? pj::k_encode_model<PJ_MODEL_USER, true, ENC_MODEL_BT, ENC_MODEL_TILE>
-                                    : pj::k_encode_model<PJ_MODEL_USER, false, ENC_MODEL_BT, ENC_MODEL_TILE>);
+    const bool pretty = P.format == PJ_FORMAT_PRETTY, size = P.cap == 0;
+    const auto kern = P.model == PJ_MODEL_ORDER ? model_kernel<PJ_MODEL_ORDER>(pretty, size)
+                                                : model_kernel<PJ_MODEL_USER>(pretty, size);
     hipLaunchKernelGGL(kern, dim3((unsigned)nblk), dim3(ENC_MODEL_BT), 0, st, P);
     return hipGetLastError();
 }

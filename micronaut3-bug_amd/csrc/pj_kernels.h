@@ -196,7 +196,7 @@ hipError_t pj_launch_encode_big(const EncParams &P, bool full, hipStream_t st);
 int pj_encode_block_records(bool nested);
 // one thread per output record (pretty output, or a selection of records)
 hipError_t pj_launch_encode_rows(const EncParams &P, bool pretty, hipStream_t st);
-hipError_t pj_launch_pretty_size(const EncParams &P, hipStream_t st);   // the total alone
+hipError_t pj_launch_rows_size(const EncParams &P, bool pretty, hipStream_t st);   // the total alone
 // pretty output of nested records through the tiled encode (blocks of
 // pj_encode_pretty_tile_records() records)
 hipError_t pj_launch_encode_pretty(const EncParams &P, hipStream_t st);
@@ -209,7 +209,7 @@ int pj_encode_model_records();
 hipError_t pj_launch_decode_model(const ModelDecParams &P, int model, hipStream_t st);
 int pj_decode_model_block();
 int pj_encode_pretty_records();
-int pj_encode_pretty_size_records();
+int pj_encode_rows_size_records();
 hipError_t pj_launch_put_bytes(uint8_t *out, uint32_t w, int k, hipStream_t st);
 hipError_t pj_launch_dec_index(const DecParams &P, hipStream_t st);
 hipError_t pj_launch_dec_parse(const DecParams &P, hipStream_t st);

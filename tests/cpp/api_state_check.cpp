@@ -6,7 +6,8 @@
 //     larger blocks whichever are used;
 //   * encode: the words that a pass starts from zero are zero at its launch,
 //     also when the scratch grew in between and its new memory has the old
-//     address; large records get a full grid where their count is not known.
+//     address; large records get a full grid where their count is not known;
+//     a call without room for output launches the size alone.
 #include <sys/mman.h>
 
 #include <cstdio>
@@ -94,7 +95,7 @@ int pj_decode_model_block() { return 128; }
 int pj_encode_block_records(bool nested) { return nested ? 96 : 256; }
 int pj_encode_model_records() { return 512; }
 int pj_encode_pretty_records() { return 256; }
-int pj_encode_pretty_size_records() { return 512; }
+int pj_encode_rows_size_records() { return 512; }
 int pj_encode_pretty_tile_records() { return 64; }
 uint64_t pj_select_blocks(uint64_t n) { return (n + 4095) / 4096; }
 hipError_t pj_noalloc_scratch_init(int, uint64_t **p) { *p = nullptr; return hipSuccess; }
@@ -161,6 +162,16 @@ hipError_t pj_launch_encode_big(const EncParams &, bool full, hipStream_t) {
     big_grids.push_back(full);
     return hipSuccess;
 }
+static int size_launches;
+hipError_t pj_launch_rows_size(const EncParams &P, bool, hipStream_t) {
+    size_launches++;
+    *P.total = 100;
+    return hipSuccess;
+}
+hipError_t pj_launch_select_status(const EncParams &P, uint32_t, uint64_t *, hipStream_t) {
+    *P.total = P.c.n_pets;
+    return hipSuccess;
+}
 hipError_t pj_launch_encode_measure(const EncParams &P, hipStream_t) { *P.ticket = 1; return hipSuccess; }
 #define UNUSED_LAUNCH(name, ...) \
     hipError_t name(__VA_ARGS__) { expect(false, #name " launched", where_now); return hipSuccess; }
@@ -169,11 +180,9 @@ UNUSED_LAUNCH(pj_launch_put_bytes, uint8_t *, uint32_t, int, hipStream_t)
 UNUSED_LAUNCH(pj_launch_copy_pieces, const CopyPieces &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_arr_frame, const DecParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_rows, const EncParams &, bool, hipStream_t)
-UNUSED_LAUNCH(pj_launch_pretty_size, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_pretty, const EncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_encode_model, const ModelEncParams &, hipStream_t)
 UNUSED_LAUNCH(pj_launch_decode_model, const ModelDecParams &, int, hipStream_t)
-UNUSED_LAUNCH(pj_launch_select_status, const EncParams &, uint32_t, uint64_t *, hipStream_t)
 
 // ------------------------------------------------------------------ checks
 static uint64_t dev[64];                 // stands for every column: never read
@@ -291,6 +300,28 @@ static void large_record_launches() {
     pj_destroy(ctx);
 }
 
+// Selections and flat pretty records: a call without room for output launches
+// the size alone (the writer is an UNUSED_LAUNCH).
+static void size_without_room(pj_ctx *ctx) {
+    pj_pet_columns c;
+    std::memset(&c, 0, sizeof c);
+    c.id = reinterpret_cast<int64_t *>(dev);
+    c.name_off = dev;
+    c.name_bytes = reinterpret_cast<uint8_t *>(dev);
+    c.n_pets = 1000;
+    uint64_t len = 0, m = 0;
+    for (int format : {PJ_FORMAT_ARRAY, PJ_FORMAT_NDJSON, PJ_FORMAT_PRETTY}) {
+        where_now = "selection, no room";
+        size_launches = 0;
+        expect(pj_encode_by_status_device(ctx, &c, 1, format, nullptr, 0, &len, &m) == PJ_ERR_CAPACITY && len == 100 &&
+                   m == 1000 && size_launches == 1, "the size alone", where_now);
+    }
+    where_now = "flat pretty, no room";
+    size_launches = 0;
+    expect(pj_encode_device(ctx, &c, PJ_FORMAT_PRETTY, nullptr, 0, &len) == PJ_ERR_CAPACITY && len == 100 &&
+               size_launches == 1, "the size alone", where_now);
+}
+
 int main() {
     large_record_launches();
     pj_status s;
@@ -298,6 +329,7 @@ int main() {
     if (!ctx) { std::printf("FAIL: no context\n"); return 1; }
     scratch_zero(ctx);
     span_guard(ctx);
+    size_without_room(ctx);
     pj_destroy(ctx);
     if (fails) return 1;
     std::printf("api state checks passed\n");

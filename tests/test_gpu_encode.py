@@ -2,6 +2,7 @@
 restatement on the same seeded records, for every configuration, both
 framings and every inclusion option, plus edge cases (empty input, one
 record, misaligned columns, capacity overflow)."""
+import ctypes as C
 import hashlib
 
 import numpy as np
@@ -628,6 +629,26 @@ def test_encode_pretty_size_around_its_blocks(codec, n):
     for config in (2, 3):
         cols = pj.generate(config, n, seed=n)
         assert codec.encode_size(cols.to_device(), pj.FORMAT_PRETTY) == len(orc.encode(cols, pj.FORMAT_PRETTY))
+
+
+@pytest.mark.parametrize("fmt", [pj.FORMAT_ARRAY, pj.FORMAT_NDJSON, pj.FORMAT_PRETTY])
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 1025, 70_000])
+def test_size_without_room(codec, n, fmt):
+    """A call with no room for output only reports the size: selections, flat
+    and nested (skewed records in the small sets), and the pretty encode."""
+    size, sel = C.c_uint64(0), C.c_uint64(0)
+    for config in (2, 3, 5) if n < 2000 else (2, 3):
+        cols = pj.generate(config, n, seed=n)
+        dev = cols.to_device()
+        torch.cuda.synchronize()
+        s = dev.struct()
+        for mask in (0, 2, 15):
+            want, m = orc.encode_by_status(cols, mask, fmt)
+            rc = codec.L.pj_encode_by_status_device(codec.ctx, C.byref(s), mask, fmt, None, 0, C.byref(size), C.byref(sel))
+            assert rc == (pj.PJ_ERR_CAPACITY if want else pj.PJ_OK)
+            assert (size.value, sel.value) == (len(want), m), (config, mask)
+        rc = codec.L.pj_encode_device(codec.ctx, C.byref(s), fmt, None, 0, C.byref(size))
+        assert rc == pj.PJ_ERR_CAPACITY and size.value == len(orc.encode(cols, fmt)), config
 
 
 @pytest.mark.parametrize("fmt", [pj.FORMAT_ARRAY, pj.FORMAT_NDJSON, pj.FORMAT_PRETTY])

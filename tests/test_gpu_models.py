@@ -3,6 +3,7 @@ byte-identical to the CPU restatement, and pj_decode_model_device gives the
 restatement's columns, error indices and codes, on the hand-written vectors,
 seeded random records in every framing and inclusion mode, and mutated
 lines."""
+import ctypes as C
 import random
 
 import numpy as np
@@ -275,3 +276,16 @@ def test_model_encode_tile_runs_match_oracle(codec, n, fmt):
             assert (host[cap:] == 0xEE).all()
             w = host[:cap] != 0xEE
             assert (host[:cap][w] == np.frombuffer(ref, np.uint8)[:cap][w]).all()
+
+
+@pytest.mark.parametrize("model", [pj.MODEL_ORDER, pj.MODEL_USER])
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 1025, 70_000])
+def test_model_size_without_room(codec, n, model):
+    """A model encode with no room for output only reports the size."""
+    cols = pj.generate_model(model, n, seed=n, null_rate=0.2)
+    dev = cols.to_device()
+    torch.cuda.synchronize()
+    s, size = dev.struct(), C.c_uint64(0)
+    for fmt in (pj.FORMAT_ARRAY, pj.FORMAT_NDJSON, pj.FORMAT_PRETTY):
+        rc = codec.L.pj_encode_model_device(codec.ctx, model, C.byref(s), fmt, None, 0, C.byref(size))
+        assert rc == pj.PJ_ERR_CAPACITY and size.value == len(orc.encode_model(cols, fmt)), fmt
