@@ -191,9 +191,10 @@ void        pj_default_options(pj_options *opt);
 pj_status   pj_set_options(pj_ctx *ctx, const pj_options *opt);
 /* Thread-local text of the last failure on this thread. */
 const char *pj_last_error(void);
-/* Duration (ms, device clock stamps at the start of each launch and of the
- * one that ends the call) of the last call's kernels:
- * index 0 = whole device pipeline, 1.. = individual kernels in launch order.
+/* Durations (ms) of the last call's kernels, from device clock stamps:
+ * index 0 = whole device pipeline, 1.. = its stages in launch order, each from
+ * the start of its first launch to the start of the next stage's (or of the
+ * launch that ends the call), so a stage of several kernels is one entry.
  * Returns the number of entries written. */
 int         pj_last_timings(const pj_ctx *ctx, float *ms, int cap);
 
@@ -201,7 +202,8 @@ int         pj_last_timings(const pj_ctx *ctx, float *ms, int cap);
 /* Serialise n_pets records (ObjectMapper.writeValueAsBytes(List<Pet>) for
  * PJ_FORMAT_ARRAY).  Device pointers.  *out_len receives the exact encoded
  * size; when it exceeds out_cap nothing past out_cap is written and
- * PJ_ERR_CAPACITY is returned. */
+ * PJ_ERR_CAPACITY is returned (what lies before out_cap is then no text to
+ * use: a record may be missing or cut). */
 pj_status pj_encode_device(pj_ctx *ctx, const pj_pet_columns *cols, int format,
                            uint8_t *out, uint64_t out_cap, uint64_t *out_len);
 /* Exact encoded size only (length pass). */

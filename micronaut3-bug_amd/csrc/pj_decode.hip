@@ -1457,7 +1457,7 @@ struct FLineT {
             q += k;
             const uint32_t c = (uint32_t)((m0 ? x0 : x1) >> (8 * (k & 7))) & 0xFF;
             if (c == '"') break;
-            // an escape, a UTF-8 sequence or an error: out of line
+            // an escape, a UTF-8 sequence or an error
             const uint32_t st = str_step((const PJ_LDS uint8_t *)s, n, q, c, ld8(q));
             if (!st) {
                 r.err = PJ_REC_STRING;
@@ -2107,10 +2107,10 @@ __device__ __forceinline__ int fline(const FL &F, LineRec &R, const BlockCols *W
 #undef FL_UNKNOWN
 
 // ------------------------------------------------- the validating walk
-// What fline<false, FLine, true> does (validate, measure, record the tape),
-// written for the least instructions and the fewest dependent LDS reads per
-// line, as it is the decode's longest kernel (bound by instruction issue and
-// LDS latency at two and a half waves per SIMD):
+// Pass 0 of fline (validate and measure) that also records the tape, written
+// for the least instructions and the fewest dependent LDS reads per line, as
+// it is the decode's longest kernel (bound by instruction issue and LDS
+// latency at two and a half waves per SIMD):
 //   * an integer is three loads at once for its digits and then its last
 //     sixteen digits and what follows it, again at once: no power-of-ten
 //     loops, no byte reads;

@@ -291,12 +291,6 @@ __device__ __forceinline__ uint64_t str_stop8(uint64_t x) {
     const uint64_t b = x ^ (0x5C * ONES);
     return (((b - ONES) & ~b) | ((x ^ QFLIP) - 0x21 * ONES) | x) & (0x80 * ONES);
 }
-// The same for '"' and '\\' only.
-__device__ __forceinline__ uint64_t quote_bs8(uint64_t x) {
-    constexpr uint64_t ONE = 0x0101010101010101ull;
-    const uint64_t q = x ^ (0x22 * ONE), b = x ^ (0x5C * ONE);
-    return (((q - ONE) & ~q) | ((b - ONE) & ~b)) & (0x80 * ONE);
-}
 // Continuation bytes a UTF-8 lead byte c takes under jackson's lead classes
 // (C0-DF one, E0-EF two, F0-F7 three), given x = the 8 bytes from the lead
 // byte on; 0 if c is no lead byte (a control, a stray continuation byte,

@@ -2132,8 +2132,8 @@ __device__ __forceinline__ void emit_runs(const P &p, RunTile<BT, TILE> &sh, uin
 // (P.sel: output record j is column record sel[j]; compact or pretty).  Each
 // thread measures its record from global memory, a block scan places the
 // records, and they leave in runs through the tile (emit_runs).  Bound by the
-// latency of each record's reads.  A third of 2M nested records by status: 0.51 -> 0.43 ms
-// against 32-byte sectors stored by each thread; 2M flat records pretty:
+// latency of each record's reads.  A third of 2M nested records by status:
+// 0.51 -> 0.42 ms against 32-byte sectors stored by each thread; 2M flat records pretty:
 // 0.27 -> 0.16 ms.  Without a tile (TILE 0): the size alone.
 template <int BT, bool PRETTY, int TILE>
 __global__ __launch_bounds__(BT, TILE ? 4 : 1) void k_encode_rows(EncParams P) {
@@ -2320,7 +2320,7 @@ __device__ __forceinline__ void m_rec(S &s, const ModelEncParams &P, uint64_t i,
 // loaded once, measured, placed by a block scan and written in runs through
 // the tile (TILE 0: the size alone).  Bound by the instructions of the two
 // passes over each record and by the latency of its scattered string reads.
-// 1M Orders (178 MB moved) 0.189 -> 0.103 ms and 1M Users 0.344 -> 0.237 ms
+// 1M Orders (178 MB moved) 0.189 -> 0.089 ms and 1M Users 0.344 -> 0.214 ms
 // against a second pass that loaded the values again and stored 32-byte
 // sectors from each thread.
 template <int MODEL, bool PRETTY, int BT, int TILE>
@@ -2605,7 +2605,8 @@ hipError_t pj_launch_select_status(const EncParams &P, uint32_t mask, uint64_t *
 }
 
 // Blocks of 512 records with a 78 KiB tile: 16 waves per CU in two
-// workgroups.  1M Orders 0.103 ms, 1M Users 0.237 ms; 256 records and 39 KiB
+// workgroups.  All by runs (emit_runs' vote, which came later, spares spills:
+// 0.089 / 0.214): 1M Orders 0.103 ms, 1M Users 0.237 ms; 256 records and 39 KiB
 // 0.107 / 0.237, 256 and 31 KiB 0.112 / 0.262, 128 and 19 KiB 0.130 / 0.236
 // (more look-backs chained), 256 and 39 KiB without the 128-VGPR cap that
 // four waves per SIMD need 0.108 / 0.256.  A call without room for output asks

@@ -968,8 +968,7 @@ __device__ __forceinline__ void m_copy_esc(const MLds &L, uint32_t q, uint32_t l
 // Bound by the scattered string stores (16-byte stores at any address).  1M
 // Users 0.61 -> 0.25 ms with the strings copied straight from the tile and
 // one exchange for all scans instead of two barriers per counter.  (Capped
-// at 168 VGPRs instead of its 232 it spills 82: 0.40 against 0.29 ms before the
-// escapes left eight bytes at a time.)
+// at 168 VGPRs instead of its 232: 0.36 against 0.25 ms.)
 // ALL_TAPED: every record is on the tape (the launcher's rule), so the
 // kernel holds no reader and keeps its registers for the copies.
 template <int MODEL, int BT, int TILE, bool ALL_TAPED>
