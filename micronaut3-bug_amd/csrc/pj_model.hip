@@ -745,8 +745,11 @@ template <int MODEL, class B> __device__ __forceinline__ int m_line_fast(const B
 // A block's records, staged: the input bytes [g0, a1) (g0 = the first
 // record's start rounded down to 16 bytes, a1 = the last record's end) in
 // LDS when they fit the tile, read with 16-byte loads, eight per thread in
-// flight (single bytes at the input's end).  Every record is then read from LDS; a block that does not fit reads
-// from global memory.
+// flight (single bytes at the input's end).  Every record is then read from
+// LDS; a block that does not fit reads from global memory.  The loads in flight
+// are of a plain vector type: an array of the runtime's uint4 class stayed in
+// scratch memory, 128 bytes per thread written and read back (4M Orders:
+// k_mdec_count 653 -> 350 us, k_mdec_write 530 -> 235; 4M Users: 873 -> 460, 807 -> 387).
 struct MStage {
     const uint8_t *tile;
     uint64_t g0;
@@ -756,6 +759,7 @@ struct MStage {
     }
 };
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 template <int BT, int TILE>
 __device__ __forceinline__ MStage m_stage(const ModelDecParams &P, uint8_t *tile, uint64_t b) {
     const uint64_t l0 = b * BT, l1 = min(l0 + BT, P.lines);
@@ -766,13 +770,13 @@ __device__ __forceinline__ MStage m_stage(const ModelDecParams &P, uint8_t *tile
         const uint32_t whole = (uint32_t)min((uint64_t)nch, (P.len - g0) >> 4);   // chunks that lie in the input whole
         constexpr int U = 8;                     // loads of a thread in flight together
         for (uint32_t c = threadIdx.x; c < whole; c += U * BT) {
-            uint4 v[U];
+            u32x4 v[U];
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (c + u * BT < whole) v[u] = *reinterpret_cast<const uint4 *>(P.in + g0 + 16ull * (c + u * BT));
+                if (c + u * BT < whole) v[u] = *reinterpret_cast<const u32x4 *>(P.in + g0 + 16ull * (c + u * BT));
 #pragma unroll
             for (int u = 0; u < U; u++)
-                if (c + u * BT < whole) reinterpret_cast<uint4 *>(tile)[c + u * BT] = v[u];
+                if (c + u * BT < whole) reinterpret_cast<u32x4 *>(tile)[c + u * BT] = v[u];
         }
         if (whole < nch && threadIdx.x < 16) {   // the input's last bytes, one by one
             const uint64_t g = g0 + 16ull * whole + threadIdx.x;
@@ -836,7 +840,7 @@ template <int MODEL> constexpr bool m_counter(int k) {
 }
 
 // Bound by the instructions of the walk (every lane its own record in LDS):
-// 1M Users (171 MB) 2.86 -> 0.25 ms, 1M Orders (123 MB) 0.77 -> 0.13 ms
+// 1M Users (171 MB) 2.86 -> 0.19 ms, 4M Orders (533 MB) 1.01 -> 0.35 ms
 // against the form that recursed from both outcomes of a property's test
 // (the User text holds escapes in one record of four and a null property in
 // more than half of them).
@@ -966,9 +970,9 @@ __device__ __forceinline__ void m_copy_esc(const MLds &L, uint32_t q, uint32_t l
 }
 
 // Bound by the scattered string stores (16-byte stores at any address).  1M
-// Users 0.61 -> 0.25 ms with the strings copied straight from the tile and
+// Users 0.61 -> 0.16 ms with the strings copied straight from the tile and
 // one exchange for all scans instead of two barriers per counter.  (Capped
-// at 168 VGPRs instead of its 232: 0.36 against 0.25 ms.)
+// at 168 VGPRs instead of its 232 it spills 82: 0.26 against 0.16 ms.)
 // ALL_TAPED: every record is on the tape (the launcher's rule), so the
 // kernel holds no reader and keeps its registers for the copies.
 template <int MODEL, int BT, int TILE, bool ALL_TAPED>
@@ -1095,8 +1099,8 @@ hipError_t pj_launch_decode_model(const ModelDecParams &P, int model, hipStream_
                        P);
     hipLaunchKernelGGL(pj::k_mdec_scan_tops, dim3(1), dim3(pj::MD_TOPS), 0, st, P);
     // every record is on the tape when there is one and no record can be
-    // 4 GiB long; the kernel without a reader then writes them (1M Users: 0.29
-    // against 0.36 ms with the reader in it)
+    // 4 GiB long; the kernel without a reader then writes them (4M Orders:
+    // 0.235 against 0.387 ms with the reader in it, 4M Users 0.387 / 0.397)
     const bool all_taped = P.tape && P.len < (1ull << 32);
     const auto write = model == PJ_MODEL_ORDER
                            ? (all_taped ? pj::k_mdec_write<PJ_MODEL_ORDER, MDEC_BT, MDEC_TILE, true>
